@@ -74,6 +74,8 @@ constexpr int kMaxTileRows = 64;
 constexpr int kMaxTileRowsLong = 128;
 constexpr int kFwdTileRows128W = 24;
 constexpr int kMinTileRows = 8;
+// The slabs' byte extents, rounded up to whole words, must be 32-bit counts.
+constexpr int64_t kMaxSlabBytes = (int64_t(1) << 32) - 3;
 static_assert(kMaxTileRows + 2 * (kMaxFastW - 1) <= kRowIds, "tile and halos must fit one RowIds");
 static_assert(kMaxFastW <= kMaxTileRows, "the longest tile must be longer than every window");
 
@@ -175,8 +177,7 @@ Tiling fast_tiling(int64_t B, int64_t T, int64_t D, int vec, int nw, int lmin, i
                    int64_t target_waves, int override_rows,
                    int64_t min_time_wg = kMinTimeWorkgroups) {
   Tiling t{};
-  const int64_t G = D / vec;
-  t.nGW = (int32_t)cdiv(G, 64);
+  t.nGW = (int32_t)cdiv(cdiv(D, vec), 64);
   int L = lmax;
   if (override_rows > 0) {
     L = override_rows;
@@ -225,7 +226,7 @@ int fwd_cpl_small(int x_dt) {
 
 // Channels per lane and waves per workgroup of the vectorised forward for a shape: CPL, or
 // CPL_SMALL when the CPL grid falls short of kTargetWaves waves even with its shortest tiles (or
-// dim is not a multiple of CPL). Measured (forward alone, bf16, W=4, 2 against 4 channels): B=4
+// dim has fewer than CPL channels). Measured (forward alone, bf16, W=4, 2 against 4 channels): B=4
 // D=1024 T=512 5.23 -> 4.68 us, T=2048 8.47 -> 8.11; B=16 D=2048 chunks of T=256 9.36 -> 9.04 us
 // per call, decode steps 2.56 -> 2.53. Grids that reach the target keep 4 channels (benchmark shape
 // 29.5 against 31.8 us; B=2 T=8192 D=1024 13.3 against 14.0). fp32 x follows the same rule in both
@@ -248,7 +249,7 @@ FastShape fwd_shape(int x_dt, int64_t B, int64_t T, int64_t D, int64_t W) {
     sh.cpl = fwd_cpl_small(x_dt);
   } else if (x_dt != CCV1D_F64 && B > 0 && T > 0 && D > 0) {
     const Tiling t = fwd_tiling_for(B, T, D, W, sh.cpl, sh.nw, false);
-    if (D % sh.cpl || B * t.nT * t.nGW < kTargetWaves || (esize(x_dt) == 2 && t.L < kFwdShortTile))
+    if (D < sh.cpl || B * t.nT * t.nGW < kTargetWaves || (esize(x_dt) == 2 && t.L < kFwdShortTile))
       sh.cpl = fwd_cpl_small(x_dt);
   }
   return sh;
@@ -322,8 +323,10 @@ int cpl_wide(int x_dt) {
 }
 
 // Channels per lane and waves per workgroup of the vectorised backward for a shape: CPL_WIDE from
-// kBwdWideW up (register budget), and below it when the 4-channel grid is small (above) or dim is
-// not a multiple of 4; CPL otherwise; kCplLong from kBwdLongW up.
+// kBwdWideW up (register budget), and below it when the 4-channel grid is small (above) or dim has
+// fewer than 4 channels; CPL otherwise; kCplLong from kBwdLongW up. Rows whose length 4 channels do not
+// divide follow the same rule (fwd+bwd B=8 T=2047 D=5375 W=4: 206 us with 4 channels in both passes,
+// 229 with 2; forward alone B=4 T=20001 D=1501: 136 against 168).
 FastShape bwd_shape(int x_dt, int64_t B, int64_t T, int64_t D, int64_t W) {
   FastShape sh = shape_of<BwdCfg>(x_dt);
   if (W >= kBwdLongW) {
@@ -332,7 +335,7 @@ FastShape bwd_shape(int x_dt, int64_t B, int64_t T, int64_t D, int64_t W) {
     sh.cpl = cpl_wide(x_dt);
   } else if (x_dt != CCV1D_F64 && B > 0 && T > 0 && D > 0) {
     const Tiling t = bwd_tiling_for(B, T, D, W, x_dt, sh.cpl, sh.nw, false);
-    if (D % sh.cpl || t.L < kBwdNarrowMinRows || B * t.nT * t.nGW < kTargetWaves)
+    if (D < sh.cpl || t.L < kBwdNarrowMinRows || B * t.nT * t.nGW < kTargetWaves)
       sh.cpl = cpl_wide(x_dt);
   }
   return sh;
@@ -395,33 +398,40 @@ int check_common(const void* x, int64_t s_xb, int64_t s_xt, int x_dt, const void
   return CCV1D_OK;
 }
 
-// The vectorised kernels read and write rows of `cpl` channels per lane: dim a multiple of cpl, the
-// base and the strides aligned to the access width, and every byte offset inside one batch slab
-// below 2^32 (they address rows through 32-bit buffer offsets).
-bool rows_ok(int x_dt, int cpl, int64_t T, int64_t D, const void* p, int64_t s_b, int64_t s_t) {
+// The vectorised kernels read and write rows of `cpl` channels per lane: at least cpl channels, the
+// base on an element, and every byte offset inside one batch slab below 2^32 (they address rows
+// through 32-bit buffer offsets).
+bool rows_ok(int x_dt, int cpl, int64_t T, int64_t D, const void* p, int64_t s_t) {
   const int64_t esz = esize(x_dt);
+  if (D < cpl || reinterpret_cast<uintptr_t>(p) % (uintptr_t)esz) return false;
+  return ((T - 1) * s_t + D) * esz < kMaxSlabBytes;
+}
+
+// Whether every row of an array starts on a multiple of the `cpl` channels a lane moves.
+bool rows_aligned(int x_dt, int cpl, int64_t D, const void* p, int64_t s_b, int64_t s_t) {
   if (D % cpl || s_b % cpl || s_t % cpl) return false;
-  if (reinterpret_cast<uintptr_t>(p) % (uintptr_t)(cpl * esz)) return false;
-  return ((T - 1) * s_t + D) * esz < (int64_t(1) << 32);
+  return reinterpret_cast<uintptr_t>(p) % (uintptr_t)(cpl * esize(x_dt)) == 0;
 }
 
 bool aligned_to(const void* p, int64_t bytes) {
   return (reinterpret_cast<uintptr_t>(p) % (uintptr_t)bytes) == 0;
 }
 
-// A channel slice of a wider channels-last tensor (strides other than the contiguous (T * D, D))
-// whose rows do not all start on a 128-byte line: each row's first and last lines, and the lines
-// where neighbouring wave columns meet, are shared with other columns (TileCoord's col_fast).
-bool straddling_slice(const void* p, int64_t s_b, int64_t s_t, int64_t B, int64_t T, int64_t D,
-                      int es) {
-  if ((s_t == D || T == 1) && (s_b == T * D || B == 1)) return false;
-  const bool aligned = aligned_to(p, 128) && (T == 1 || (s_t * es) % 128 == 0) &&
-                       (B == 1 || (s_b * es) % 128 == 0);
-  return !aligned;
+// Whether rows start off the `bytes` boundaries: with 128, the first and last lines of a row, and the
+// lines where neighbouring wave columns meet, are shared with other columns (TileCoord's col_fast).
+// Such rows are channel slices of a wider tensor, or contiguous rows of an odd length. The second
+// kind measured with the column-fastest order (bf16 W=4, time-fastest first): fwd+bwd B=4 T=5001
+// D=1501 92.5 -> 86.5 us, D=1500 89.0 -> 82.8, B=8 T=2047 D=5375 237 -> 206, B=1 T=4001 D=2001 27.0
+// -> 23.5; forward alone B=4 T=20001 D=1501 158 -> 136; D=1504 (rows on 64 bytes) even.
+bool rows_off(const void* p, int64_t s_b, int64_t s_t, int64_t B, int64_t T, int es, int bytes) {
+  return !(aligned_to(p, bytes) && (T == 1 || (s_t * es) % bytes == 0) &&
+           (B == 1 || (s_b * es) % bytes == 0));
 }
 
+// Extent of one batch slab as the buffer resources' limit: its bytes rounded up to whole words, so
+// that a last word which starts inside an odd count of 16-bit elements is inside the limit.
 uint32_t slab_bytes(int x_dt, int64_t T, int64_t D, int64_t s_t) {
-  return (uint32_t)(((T - 1) * s_t + D) * esize(x_dt));
+  return (uint32_t)((((T - 1) * s_t + D) * esize(x_dt) + 3) & ~int64_t(3));
 }
 
 bool fast_dtype(int x_dt, int64_t W) { return W <= kMaxFastW && x_dt != CCV1D_F64; }
@@ -491,15 +501,16 @@ int fwd_entry(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype
   if (B * D == 0) return CCV1D_OK;
   const int fcpl = fwd_shape(x_dtype, B, T, D, W).cpl;
   const bool fast = T > 0 && fast_dtype(x_dtype, W) &&
-                    rows_ok(x_dtype, fcpl, T, D, x, x_stride_b, x_stride_t) &&
-                    rows_ok(x_dtype, fcpl, T, D, out, T * D, D) &&
-                    (!final_states || aligned_to(final_states, fcpl * esize(x_dtype)));
+                    rows_ok(x_dtype, fcpl, T, D, x, x_stride_t) &&
+                    rows_ok(x_dtype, fcpl, T, D, out, D) &&
+                    (!final_states || aligned_to(final_states, esize(x_dtype)));
   Tiling tl{};
   if (T > 0) {
     if (fast) {
       tl = fwd_fast_tiling(B, T, D, W, x_dtype, seq_idx != nullptr);
       tl.col_fast = W <= kColFastMaxW &&
-                    straddling_slice(x, x_stride_b, x_stride_t, B, T, D, esize(x_dtype));
+                    (rows_off(x, x_stride_b, x_stride_t, B, T, esize(x_dtype), 128) ||
+                     rows_off(out, T * D, D, B, T, esize(x_dtype), 128));
     } else {
       tl = generic_tiling(T);
       if (B * tl.nT >= (int64_t(1) << 31) || cdiv(D, 64) > 65535)
@@ -679,10 +690,10 @@ BwdPath bwd_path(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dt
                  int64_t W) {
   BwdPath r;
   const int bcpl = bwd_shape(x_dtype, B, T, D, W).cpl;
-  r.fast = fast_dtype(x_dtype, W) && rows_ok(x_dtype, bcpl, T, D, x, x_stride_b, x_stride_t) &&
-           rows_ok(x_dtype, bcpl, T, D, dout, dout_stride_b, dout_stride_t) &&
-           rows_ok(x_dtype, bcpl, T, D, dx, dx_stride_b, dx_stride_t) &&
-           (!dfinal_states || aligned_to(dfinal_states, bcpl * esize(x_dtype))) && ws_aligned;
+  r.fast = fast_dtype(x_dtype, W) && rows_ok(x_dtype, bcpl, T, D, x, x_stride_t) &&
+           rows_ok(x_dtype, bcpl, T, D, dout, dout_stride_t) &&
+           rows_ok(x_dtype, bcpl, T, D, dx, dx_stride_t) &&
+           (!dfinal_states || aligned_to(dfinal_states, esize(x_dtype))) && ws_aligned;
   if (r.fast) {
     r.tl = bwd_fast_tiling(B, T, D, W, x_dtype, seq);
     r.rows = B * r.tl.nTB;
@@ -795,11 +806,14 @@ int plan_bwd(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype,
     p.y_bytes = slab_bytes(x_dtype, T, D, dout_stride_t);
     p.o_bytes = slab_bytes(x_dtype, T, D, dx_stride_t);
     const int es = esize(x_dtype);
-    const bool dx_straddles = straddling_slice(dx, dx_stride_b, dx_stride_t, B, T, D, es);
     p.tl.col_fast = W <= kColFastMaxW &&
-                    (dx_straddles || straddling_slice(x, x_stride_b, x_stride_t, B, T, D, es) ||
-                     straddling_slice(dout, dout_stride_b, dout_stride_t, B, T, D, es));
-    p.dx_nt = dx_straddles;
+                    (rows_off(dx, dx_stride_b, dx_stride_t, B, T, es, 128) ||
+                     rows_off(x, x_stride_b, x_stride_t, B, T, es, 128) ||
+                     rows_off(dout, dout_stride_b, dout_stride_t, B, T, es, 128));
+    // Plain non-temporal dx stores where rows also start inside half-lines (BwdCfg::DXST_STREAM):
+    // D=1501 88.6 -> 86.5 us, B=8 T=2047 D=5375 215.5 -> 206; rows on 64 bytes keep sc1 (D=1504 69.3
+    // -> 66.8).
+    p.dx_nt = rows_off(dx, dx_stride_b, dx_stride_t, B, T, es, 64);
   } else if (path.rows >= (int64_t(1) << 31) || cdiv(D, 64) > 65535) {
     return fail(CCV1D_ERR_UNSUPPORTED, "shape too large for the generic kernel");
   }
@@ -876,9 +890,21 @@ size_t ccv1d_bwd_workspace_bytes_for(const void* x, int64_t x_stride_b, int64_t 
   const int64_t B = batch, T = seqlen, D = dim, W = width;
   if (B <= 0 || T <= 0 || D <= 0 || W < 2 || !valid_dt(x_dtype)) return 0;
   if (x_stride_b < 0 || x_stride_t < 0 || dout_stride_b < 0 || dout_stride_t < 0) return 0;
-  return bwd_path(x, x_stride_b, x_stride_t, x_dtype, seq_idx != nullptr, dout, dout_stride_b,
-                  dout_stride_t, dfinal_states, dx, T * D, D, true, B, T, D, W)
-      .need;
+  const size_t need = bwd_path(x, x_stride_b, x_stride_t, x_dtype, seq_idx != nullptr, dout,
+                               dout_stride_b, dout_stride_t, dfinal_states, dx, T * D, D, true, B,
+                               T, D, W)
+                          .need;
+  // Rows that do not start on the lanes' access width may be given to either family of kernels:
+  // the larger of their needs.
+  const int cpl = fast_dtype(x_dtype, W) ? bwd_shape(x_dtype, B, T, D, W).cpl : 1;
+  if (fast_dtype(x_dtype, W) &&
+      !(rows_aligned(x_dtype, cpl, D, x, x_stride_b, x_stride_t) &&
+        rows_aligned(x_dtype, cpl, D, dout, dout_stride_b, dout_stride_t) &&
+        rows_aligned(x_dtype, cpl, D, dx, T * D, D))) {
+    const size_t generic = partial_bytes(B * generic_tiling(T).nT, W, D);
+    if (generic > need) return generic;
+  }
+  return need;
 }
 
 int ccv1d_bwd(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype,

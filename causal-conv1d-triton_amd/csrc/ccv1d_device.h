@@ -66,7 +66,7 @@ struct BwdParams {
   int32_t has_bias, has_init, has_dfinal, need_dinit, silu;
   uint32_t x_bytes, y_bytes, o_bytes;  // per-batch byte extents of x, dout and dx (vectorised)
   Tiling tl;
-  // Host side: dx rows straddle 128-byte lines, stored non-temporally (BwdCfg). Kept after tl: in
+  // Host side: dx rows start inside 64-byte half-lines, stored non-temporally (BwdCfg). Kept after tl: in
   // front of it the widest kernels' kernel-argument loads left them 20-400 more SGPR spills.
   int32_t dx_nt;
 };
@@ -126,6 +126,12 @@ typedef uint32_t u32x1 __attribute__((ext_vector_type(1)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// The same words at the alignment of an element, for the accesses through plain pointers (rows and
+// states of any element address).
+template <typename V, int ALIGN> struct AlignedAs {
+  typedef V type __attribute__((aligned(ALIGN)));
+};
+
 template <int BYTES> struct RawOf;
 template <> struct RawOf<2> { using type = uint16_t; };
 template <> struct RawOf<4> { using type = u32x1; };
@@ -137,12 +143,13 @@ struct VecIO {
   static constexpr int BYTES = CPL * (int)sizeof(TX);
   static constexpr int WORDS = BYTES / 4;
   using raw = typename RawOf<BYTES>::type;
+  using mem = typename AlignedAs<raw, (int)sizeof(TX)>::type;
 
-  __device__ static __forceinline__ raw ld(const TX* p) { return *reinterpret_cast<const raw*>(p); }
-  __device__ static __forceinline__ void st(TX* p, raw v) { *reinterpret_cast<raw*>(p) = v; }
+  __device__ static __forceinline__ raw ld(const TX* p) { return *reinterpret_cast<const mem*>(p); }
+  __device__ static __forceinline__ void st(TX* p, raw v) { *reinterpret_cast<mem*>(p) = v; }
   // Non-temporal store: streamed output that no later work in the kernel reads.
   __device__ static __forceinline__ void st_nt(TX* p, raw v) {
-    __builtin_nontemporal_store(v, reinterpret_cast<raw*>(p));
+    __builtin_nontemporal_store(v, reinterpret_cast<mem*>(p));
   }
 
   __device__ static __forceinline__ void unpack(const raw v, float (&f)[CPL]) {

@@ -1,5 +1,5 @@
 // Vectorised forward and backward kernels for compile-time widths (2..kMaxFastW = 32) and
-// channels-last x whose rows are aligned to the 2-, 4-, 8- or 16-byte access of CPL channels.
+// channels-last x of at least CPL channels, whatever the alignment of its rows (lane_channel).
 //
 // Work decomposition (both passes): a lane owns CPL consecutive channels, a wave owns 64 such
 // channel vectors over a tile of L consecutive rows, and a workgroup holds NW waves on consecutive
@@ -69,6 +69,18 @@ __device__ __forceinline__ void conv_row(const float (&wv)[W][CPL], const float 
     for (int i = 0; i < CPL; ++i) z[i] = 0.0f;
   }
 }
+
+// Channel groups of a row, and the first channel of group `grp` (grp < channel_groups). Where dim is
+// not a multiple of CPL the last group is the row's last CPL channels: it shares channels with the
+// group before it, and both lanes compute and store the same bits for them. No access is wider than
+// the row, and the rows need no alignment beyond their elements': gfx950 runs 4-, 8- and 16-byte
+// accesses at any element address, and a wave's 64 of them touch one line more than aligned ones.
+// (Such rows took the scalar kernels before: B=4 T=5001 D=1501 bf16 W=4 fwd+bwd 315 -> 80 us a call, 86
+// in a graph that rotates buffers.)
+template <int CPL>
+__device__ __forceinline__ int channel_groups(int D) { return (D + CPL - 1) / CPL; }
+template <int CPL>
+__device__ __forceinline__ int lane_channel(int grp, int D) { return min(grp * CPL, D - CPL); }
 
 template <int P, int CPL>
 __device__ __forceinline__ void shift_in(float (&win)[P][CPL], const float (&v)[CPL]) {
@@ -453,8 +465,8 @@ __global__ __launch_bounds__(NW * 64, (fwd_waves_per_simd<TX, W, SEQ>())) void f
   // an activation), whatever x holds.
   const bool pad = masked && ids.all_padding(t0, t1);
   const int grp = tc.gw * 64 + lane;
-  if (grp >= p.D / CPL) return;
-  const int c0 = grp * CPL;
+  if (grp >= channel_groups<CPL>(D)) return;
+  const int c0 = lane_channel<CPL>(grp, D);
 
   const RowBuf<TX, CPL, XLD> X(static_cast<const TX*>(p.x) + (int64_t)tc.b * p.s_xb, p.x_bytes, c0,
                                p.s_xt);
@@ -652,10 +664,10 @@ __device__ __forceinline__ void bwd_tile(const BwdParams& p, float* lds, const R
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const TileCoord<(W <= kColFastMaxW)> tc(p.tl);
   const int tile = tc.tb * NW + wave;
-  const int G = p.D / CPL;
-  const int grp = tc.gw * 64 + lane;
-  const int c0 = grp * CPL;
   const int T = p.T, D = p.D;
+  const int G = channel_groups<CPL>(D);
+  const int grp = tc.gw * 64 + lane;
+  const int c0 = lane_channel<CPL>(grp, D);
   const bool active = tile < p.tl.nT && grp < G;
   const bool has_init = p.has_init;
   const int t0 = tile * p.tl.L;

@@ -54,7 +54,7 @@ template <typename TX> struct BwdCfg {
   static constexpr int XLD = kCacheNT;
   static constexpr int YLD = kCacheNT;
   static constexpr int DXST = sizeof(TX) == 2 ? kCacheSC1NT : kCacheNT;
-  // dx rows that straddle 128-byte lines (BwdParams::dx_nt; widths below kUnitWideW): plain
+  // dx rows that start inside 64-byte half-lines (BwdParams::dx_nt; widths below kUnitWideW): plain
   // non-temporal stores. Configuration 3 writing dx into the in_proj gradient (pitch 10576
   // channels), column-fastest order: 247 -> 233 us.
   static constexpr int DXST_STREAM = kCacheNT;

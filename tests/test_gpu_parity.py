@@ -1330,3 +1330,39 @@ def test_straddling_slices_match_contiguous(W):
     want = run(x, dy)
     for g, e in zip(got, want):
         assert torch.equal(g, e)
+
+
+@pytest.mark.parametrize("W", [2, 4, 5, 8, 12])
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16, torch.float32])
+def test_rows_of_any_length_and_alignment(W, xdt):
+    """Rows that the access of a lane's channels does not divide or align: the last lane of a row then
+    takes the row's last channels, which it shares with the lane before it. Channel counts around
+    one access and around a wave column, against the oracle (without the activation bit-exact);
+    then x, dout and dx as slices at an odd channel of tensors with an odd pitch, bit-identical to
+    contiguous copies (the arithmetic and the tiling do not depend on the alignment), with the
+    elements beside the dx slice untouched."""
+    from causal_conv1d_triton.fused import causal_conv1d_bwd
+
+    for D, T, act in ((2, 40, None), (3, 40, "silu"), (5, 33, None), (127, 70, "silu"),
+                      (129, 70, None), (255, 300, "silu"), (257, 300, None), (1501, 90, "silu")):
+        inp = make_inputs(17 * W + D, 2, T, D, W, xdt=xdt, init=True)
+        gpu = run_gpu(inp, act, return_final=True, dfinal=True, init_grad=True)
+        compare(gpu, oracle_ref(inp, act is not None, final=True, dfinal=True, need_dinit=True),
+                act is not None)
+    B, T, D = 2, 300, 259
+    inp = make_inputs(19 * W, B, T, D, W, xdt=xdt, init=True)
+    x, w, b, dy, s0, df = (inp[k].to(DEV) for k in ("x", "w", "b", "dy", "init", "dfinal"))
+    bx = torch.zeros(B, T, D + 14, dtype=xdt, device=DEV)
+    by = torch.zeros(B, T, D + 18, dtype=xdt, device=DEV)
+    bdx = torch.full((B, T, D + 6), 7.0, dtype=xdt, device=DEV)
+    bx[..., 5:5 + D], by[..., 1:1 + D] = x, dy
+    outs, grads = [], []
+    for xv, dyv, dxv in ((x, dy, None), (bx[..., 5:5 + D], by[..., 1:1 + D], bdx[..., 3:3 + D])):
+        with torch.no_grad():
+            outs.append(causal_conv1d_fn(xv, w, b, initial_states=s0, return_final_states=True,
+                                         activation="silu"))
+        grads.append(causal_conv1d_bwd(xv, w, b, dyv, initial_states=s0, dfinal_states=df, dx=dxv,
+                                       return_dinitial_states=True, activation="silu"))
+    for a, c in zip(outs[0] + grads[0], outs[1] + grads[1]):
+        assert torch.equal(a, c)
+    assert torch.all(bdx[..., :3] == 7.0) and torch.all(bdx[..., 3 + D:] == 7.0)
