@@ -347,7 +347,7 @@ Tiling bwd_fast_tiling(int64_t B, int64_t T, int64_t D, int64_t W, int x_dt, boo
 }
 
 // Workspace of the backward: the fp32 partial rows of dweight/dbias, (rows, W + 1, D) floats, and
-// for widths above kMaxGenericW after them, 256-byte aligned, the fp32 g buffer (B, T, D).
+// for widths above kMaxBlockW after them, 256-byte aligned, the fp32 g buffer (B, T, D).
 size_t partial_bytes(int64_t rows, int64_t W, int64_t D) {
   return (size_t)(rows * (W + 1) * D * (int64_t)sizeof(float));
 }
@@ -356,10 +356,22 @@ size_t g_buffer_bytes(int64_t B, int64_t T, int64_t D) {
 }
 size_t g_buffer_offset(size_t partials) { return (partials + 255) & ~(size_t)255; }
 
-Tiling generic_tiling(int64_t T) {
+// Tiling of the kernels without compile-time widths. Above kMaxBlockW: tiles of kGenericL rows. Up
+// to it a workgroup of the block kernels walks a segment of whole steps, and each segment reads a
+// window of rows and the weights once more (the backward also forms g of a window past its end): the
+// longest segment that still gives the grid kBlkTargetGroups workgroups, 2 per CU. A segment is
+// never shorter than kGenericL rows, so there are never more partial rows than of kGenericL-row tiles.
+constexpr int64_t kBlkTargetGroups = 512;
+constexpr int kBlkMaxRows = 2048;
+static_assert(kGenericL % kBlkStep == 0, "segments are whole steps");
+Tiling generic_tiling(int64_t B, int64_t T, int64_t D, int64_t W) {
   Tiling t{};
   t.L = kGenericL;
-  t.nT = (int32_t)cdiv(T, kGenericL);
+  if (W <= kMaxBlockW) {
+    t.L = kBlkMaxRows;
+    while (t.L > kGenericL && B * cdiv(D, 64) * cdiv(T, t.L) < kBlkTargetGroups) t.L /= 2;
+  }
+  t.nT = (int32_t)cdiv(T, t.L);
   return t;
 }
 
@@ -512,7 +524,7 @@ int fwd_entry(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype
                     (rows_off(x, x_stride_b, x_stride_t, B, T, esize(x_dtype), 128) ||
                      rows_off(out, T * D, D, B, T, esize(x_dtype), 128));
     } else {
-      tl = generic_tiling(T);
+      tl = generic_tiling(B, T, D, W);
       if (B * tl.nT >= (int64_t(1) << 31) || cdiv(D, 64) > 65535)
         return fail(CCV1D_ERR_UNSUPPORTED, "shape too large for the generic kernel");
     }
@@ -609,14 +621,14 @@ size_t ccv1d_bwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t dim, int
                                  int x_dtype) {
   const int64_t B = batch, T = seqlen, D = dim, W = width;
   if (B <= 0 || T <= 0 || D <= 0 || W < 2 || !valid_dt(x_dtype)) return 0;
-  int64_t rows = B * generic_tiling(T).nT;
+  int64_t rows = B * cdiv(T, kGenericL);  // the most segments any width takes
   if (W <= kMaxFastW && x_dtype != CCV1D_F64) {
     // With seq_idx the tiles are never longer, so its tiling has at least as many partial rows.
     const int64_t fr = B * bwd_fast_tiling(B, T, D, W, x_dtype, true).nTB;
     if (fr > rows) rows = fr;
   }
   size_t n = partial_bytes(rows, W, D);
-  if (W > kMaxGenericW) n = g_buffer_offset(n) + g_buffer_bytes(B, T, D);
+  if (W > kMaxBlockW) n = g_buffer_offset(n) + g_buffer_bytes(B, T, D);
   return n;
 }
 
@@ -665,7 +677,7 @@ struct BwdPlan {
   bool skip = false;   // dim == 0: nothing to do
   bool empty = false;  // batch == 0 or seqlen == 0: the fill path
   bool fast = false;
-  bool wide = false;   // generic path above kMaxGenericW: g goes through the workspace
+  bool wide = false;   // generic path above kMaxBlockW: g goes through the workspace
   int x_dt = 0;
   size_t g_off = 0;    // byte offset of the g buffer in the workspace (wide)
   size_t need = 0;     // workspace bytes the launches use
@@ -676,7 +688,7 @@ struct BwdPlan {
 // dfinal_states) allow them, else the generic ones.
 struct BwdPath {
   bool fast = false;
-  bool wide = false;   // generic path above kMaxGenericW: g goes through the workspace
+  bool wide = false;   // generic path above kMaxBlockW: g goes through the workspace
   Tiling tl{};
   int64_t rows = 0;    // partial rows of dweight/dbias
   size_t g_off = 0;    // byte offset of the g buffer in the workspace (wide)
@@ -698,9 +710,9 @@ BwdPath bwd_path(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dt
     r.tl = bwd_fast_tiling(B, T, D, W, x_dtype, seq);
     r.rows = B * r.tl.nTB;
   } else {
-    r.tl = generic_tiling(T);
+    r.tl = generic_tiling(B, T, D, W);
     r.rows = B * r.tl.nT;
-    r.wide = W > kMaxGenericW;
+    r.wide = W > kMaxBlockW;
   }
   r.need = partial_bytes(r.rows, W, D);
   if (r.wide) {
@@ -901,7 +913,7 @@ size_t ccv1d_bwd_workspace_bytes_for(const void* x, int64_t x_stride_b, int64_t 
       !(rows_aligned(x_dtype, cpl, D, x, x_stride_b, x_stride_t) &&
         rows_aligned(x_dtype, cpl, D, dout, dout_stride_b, dout_stride_t) &&
         rows_aligned(x_dtype, cpl, D, dx, T * D, D))) {
-    const size_t generic = partial_bytes(B * generic_tiling(T).nT, W, D);
+    const size_t generic = partial_bytes(B * cdiv(T, kGenericL), W, D);
     if (generic > need) return generic;
   }
   return need;

@@ -406,6 +406,11 @@ __device__ __forceinline__ int32_t seq_at(const int32_t* seqb, int t, int T, boo
   return seqb[t];
 }
 
+// Widths up to kMaxBlockW without a vectorised instance take the block kernels (ccv1d_block.h), whose
+// segments are whole steps of kBlkStep rows.
+constexpr int kMaxBlockW = 128;
+constexpr int kBlkStep = 64;
+
 // Maps the hardware workgroup id to a logical one so that each of the 8 XCDs (which receive
 // workgroups round-robin) runs one contiguous range of logical workgroups. Neighbouring time tiles,
 // whose halo rows overlap, then share one XCD's L2.

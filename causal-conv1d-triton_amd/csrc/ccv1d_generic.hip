@@ -1,20 +1,19 @@
-// Launchers of the scalar (any width / any alignment) kernels, the partial-sum reduction and the
-// fill kernel.
+// Launchers of the block kernels (widths up to 128), the scalar kernels (any width), the partial-sum
+// reduction and the fill kernel.
 #include <atomic>
 
-#include "ccv1d_generic.h"
+#include "ccv1d_block.h"
 #include "ccv1d_launch.h"
 
 namespace ccv1d {
 
-static_assert(kMaxGenericW <= kGenericRingW, "the ring backward covers every generic width");
-static_assert(generic_ring_bytes(kGenericRingW, 4) <= 160 * 1024, "LDS of one gfx950 CU");
+static_assert(blk_lds_bytes(kMaxBlockW, 4, true) <= 160 * 1024, "LDS of one gfx950 CU");
 
-// Dynamic LDS above the default 64 KiB per workgroup must be allowed per kernel first. Each ring
-// kernel is allowed the most any width takes (generic_ring_bytes(kGenericRingW, ...), at most the
-// 160 KiB of a gfx950 CU) once per device, on its first launch there that needs more than 64 KiB:
-// later launches, including those recorded into a captured graph, make no runtime call for it.
-// `done` is the kernel's own set of devices (bit d for device d < 64; others set it every launch).
+// Dynamic LDS above the default 64 KiB per workgroup must be allowed per kernel first. Each block
+// kernel is allowed the most any width takes (at most the 160 KiB of a gfx950 CU) once per device, on
+// its first launch there that needs more than 64 KiB: later launches, including those recorded into
+// a captured graph, make no runtime call for it. `done` is the kernel's own set of devices (bit d for
+// device d < 64; others set it every launch).
 static hipError_t allow_lds(const void* kernel, size_t bytes, size_t max_bytes,
                             std::atomic<uint64_t>& done) {
   if (bytes <= 65536) return hipSuccess;
@@ -28,30 +27,55 @@ static hipError_t allow_lds(const void* kernel, size_t bytes, size_t max_bytes,
   return e;
 }
 
+// Whether the x ring holds TX itself: 16-bit x, with initial states (if any) of the same type.
+template <typename TX, typename Params>
+static bool ring_of_tx(const Params& p) {
+  const int dt = __is_same(TX, __bf16) ? DT_BF16 : __is_same(TX, _Float16) ? DT_F16 : -1;
+  return dt >= 0 && (!p.has_init || p.i_dt == dt);
+}
+
+template <typename TX, typename E>
+static hipError_t fwd_block(const FwdParams& p, hipStream_t s) {
+  static std::atomic<uint64_t> lds_allowed{0};
+  const dim3 grid((unsigned)((int64_t)p.B * p.tl.nT), (unsigned)((p.D + 63) / 64));
+  const void* k = reinterpret_cast<const void*>(&fwd_block_kernel<TX, E>);
+  const size_t shmem = blk_lds_bytes(p.W, sizeof(E), false);
+  const hipError_t e =
+      allow_lds(k, shmem, blk_lds_bytes(kMaxBlockW, sizeof(E), false), lds_allowed);
+  if (e != hipSuccess) return e;
+  return launch(k, grid, dim3(kBlkNW * 64), shmem, s, &p);
+}
+
+template <typename TX, typename E>
+static hipError_t bwd_block(const BwdParams& p, hipStream_t s) {
+  static std::atomic<uint64_t> lds_allowed{0};
+  const dim3 grid((unsigned)((int64_t)p.B * p.tl.nT), (unsigned)((p.D + 63) / 64));
+  const void* k = reinterpret_cast<const void*>(&bwd_block_kernel<TX, E>);
+  const size_t shmem = blk_lds_bytes(p.W, sizeof(E), true);
+  const hipError_t e = allow_lds(k, shmem, blk_lds_bytes(kMaxBlockW, sizeof(E), true), lds_allowed);
+  if (e != hipSuccess) return e;
+  return launch(k, grid, dim3(kBlkNW * 64), shmem, s, &p);
+}
+
 template <typename TX>
 hipError_t launch_fwd_generic_t(const FwdParams& p, hipStream_t s) {
-  const dim3 grid((unsigned)((int64_t)p.B * p.tl.nT), (unsigned)((p.D + 63) / 64));
-  if (p.W <= kGenericRingW) {
-    static std::atomic<uint64_t> lds_allowed{0};
-    const void* k = reinterpret_cast<const void*>(&fwd_generic_ring_kernel<TX>);
-    const size_t shmem = generic_ring_bytes(p.W, 2);
-    const hipError_t e = allow_lds(k, shmem, generic_ring_bytes(kGenericRingW, 2), lds_allowed);
-    if (e != hipSuccess) return e;
-    return launch(k, grid, dim3(64), shmem, s, &p);
+  if (p.W <= kMaxBlockW) {
+    if constexpr (sizeof(TX) == 2) {
+      if (ring_of_tx<TX>(p)) return fwd_block<TX, TX>(p, s);
+    }
+    return fwd_block<TX, float>(p, s);
   }
+  const dim3 grid((unsigned)((int64_t)p.B * p.tl.nT), (unsigned)((p.D + 63) / 64));
   return launch(reinterpret_cast<const void*>(&fwd_generic_kernel<TX>), grid, dim3(64), 0, s, &p);
 }
 
-// Widths up to kMaxGenericW (<= kGenericRingW); wider ones take launch_bwd_wide_t.
+// Widths up to kMaxBlockW; wider ones take launch_bwd_wide_t.
 template <typename TX>
 hipError_t launch_bwd_generic_t(const BwdParams& p, hipStream_t s) {
-  const dim3 grid((unsigned)((int64_t)p.B * p.tl.nT), (unsigned)((p.D + 63) / 64));
-  static std::atomic<uint64_t> lds_allowed{0};
-  const void* k = reinterpret_cast<const void*>(&bwd_generic_ring_kernel<TX>);
-  const size_t shmem = generic_ring_bytes(p.W, 4);
-  const hipError_t e = allow_lds(k, shmem, generic_ring_bytes(kGenericRingW, 4), lds_allowed);
-  if (e != hipSuccess) return e;
-  return launch(k, grid, dim3(64), shmem, s, &p);
+  if constexpr (sizeof(TX) == 2) {
+    if (ring_of_tx<TX>(p)) return bwd_block<TX, TX>(p, s);
+  }
+  return bwd_block<TX, float>(p, s);
 }
 
 template <typename TX>

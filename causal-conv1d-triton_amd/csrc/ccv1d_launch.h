@@ -82,11 +82,8 @@ constexpr int kBwdWideW = 6;     // first width whose backward uses BwdCfg::CPL_
 constexpr int kFwdLongW = 17;
 constexpr int kBwdLongW = 11;
 constexpr int kCplLong = 1;
-constexpr int kMaxGenericW = 128;  // LDS rings of the generic backward (x, g, weights, dweight
-                                   // sums: 4 * W * 64 * 4 bytes + the rows' ids, 128.5 KiB at 128);
-                                   // wider backwards keep g in the workspace (bwd_g/bwd_wide)
 constexpr int kReduceNW = 16;    // waves per reduction workgroup
-constexpr int kGenericL = 64;    // rows per tile of the generic kernels
+constexpr int kGenericL = 64;    // rows per tile of the kernels above kMaxBlockW
 
 // Timing events of the calling thread (ccv1d_time_main_kernel). `pending` holds a request for the
 // thread's next entry-point call, which takes it; the call sets `armed` right before its main kernel
@@ -153,7 +150,7 @@ template <typename TX>
 hipError_t launch_fwd_generic_t(const FwdParams& p, hipStream_t s);
 template <typename TX>
 hipError_t launch_bwd_generic_t(const BwdParams& p, hipStream_t s);
-// Backward above kMaxGenericW: g to the fp32 buffer G of (batch, seqlen, dim) floats, then dx and
+// Backward above kMaxBlockW: g to the fp32 buffer G of (batch, seqlen, dim) floats, then dx and
 // the partial rows from it (the second is the main kernel for ccv1d_time_main_kernel).
 template <typename TX>
 hipError_t launch_bwd_wide_t(const BwdParams& p, float* G, hipStream_t s);

@@ -1366,3 +1366,31 @@ def test_rows_of_any_length_and_alignment(W, xdt):
     for a, c in zip(outs[0] + grads[0], outs[1] + grads[1]):
         assert torch.equal(a, c)
     assert torch.all(bdx[..., :3] == 7.0) and torch.all(bdx[..., 3 + D:] == 7.0)
+
+
+@pytest.mark.parametrize("W", [33, 49, 65, 100, 128])
+@pytest.mark.parametrize("xdt,idt", [(torch.bfloat16, torch.float32), (torch.float16, None),
+                                     (torch.float32, torch.bfloat16)])
+def test_block_kernel_edges(W, xdt, idt):
+    """Widths 33-128 around the edges of the block kernels: lengths of one step of 64 rows and beside
+    it, a channel past a group of 64, windows of whole 16-row blocks (W = 33, 49, 65) and not, 16-bit
+    x with fp32 initial states (kept in fp32), and without the activation bit-exact."""
+    for T, D, act in ((15, 64, None), (63, 65, "silu"), (64, 65, None), (65, 63, "silu"),
+                      (257, 65, None)):
+        inp = make_inputs(23 * W + T, 2, T, D, W, xdt=xdt, init=True, idt=idt)
+        gpu = run_gpu(inp, act, return_final=True, dfinal=True, init_grad=True)
+        compare(gpu, oracle_ref(inp, act is not None, final=True, dfinal=True, need_dinit=True),
+                act is not None)
+
+
+@pytest.mark.parametrize("W", [33, 72, 128])
+@pytest.mark.parametrize("seq", [False, True])
+def test_block_kernel_long_segments(W, seq):
+    """A grid whose segments are several steps long (the rings wrap), against the oracle on a subset
+    of the channels."""
+    B, T, D = 8, 2300, 584
+    ids = varlen_seq(3 * W, B, T, lo=100, hi=900) if seq else None
+    inp = make_inputs(29 * W, B, T, D, W, init=True, seq=ids)
+    gpu = run_gpu(inp, "silu", init_grad=True)
+    cols = _cols(D, 6, W)
+    compare(gpu, oracle_ref(inp, True, cols=cols, need_dinit=True), True, cols)
