@@ -375,6 +375,50 @@ Tiling generic_tiling(int64_t B, int64_t T, int64_t D, int64_t W) {
   return t;
 }
 
+// The matrix-core backward (ccv1d_mfma.h): bf16 x with silu, without seq_idx, and initial states (if
+// any) of x's dtype. Without an activation the vector kernels stay: their results are the reference's
+// operation order bit for bit.
+constexpr int64_t kMmMinW = kMaxFastW + 1;  // see ccv1d_mfma.h
+bool mfma_takes(int x_dt, int64_t D, int64_t W, bool silu, bool seq, bool init, int i_dt) {
+  return x_dt == CCV1D_BF16 && silu && !seq && W >= kMmMinW && W <= kMaxBlockW && D >= kMmCh &&
+         (!init || i_dt == x_dt);
+}
+
+// Its tiling. Every workgroup does about the same work, so what counts is how many of them one after
+// the other a CU runs (256 CUs, one at a time) and how many steps each takes: a segment and its
+// window are walked in whole steps, and a workgroup's start and end (weights, sums) cost about one
+// more. Of the segment counts that just fill 1, 2, ... rounds, the cheapest: with the longest segments
+// of 8 steps that still filled the chip, rows left over ran a second round (B=2 T=4096 D=1024 W=64
+// 170 -> 115 us, B=4 T=8192 D=1024 W=32 292 -> 212).
+constexpr int kMmMaxRounds = 8;
+Tiling mfma_tiling(int64_t B, int64_t T, int64_t D, int64_t W) {
+  Tiling t{};
+  const int64_t window = cdiv(W - 1, 16) * 16;
+  constexpr int64_t slots = 256;
+  // Only a row's first segment has a window outside x, and never more partial rows than of
+  // kGenericL-row tiles.
+  const int64_t shortest = window < kGenericL ? kGenericL : window;
+  t.nGW = (int32_t)cdiv(D, kMmCh);
+  const int64_t cols = B * t.nGW;
+  int64_t best = -1;
+  for (int64_t r = 1; r <= kMmMaxRounds; ++r) {
+    int64_t n = slots * r / cols;
+    n = n < 1 ? 1 : n;
+    const int64_t L = cdiv(cdiv(T, n), 16) * 16;
+    if (L < shortest && best >= 0) break;
+    const int64_t Ls = L < shortest ? shortest : L;
+    const int64_t groups = cols * cdiv(T, Ls);
+    const int64_t cost = cdiv(groups, slots) * (cdiv(Ls + window, kMmRows) + 1);
+    if (best < 0 || cost < best) {
+      best = cost;
+      t.L = (int32_t)Ls;
+    }
+  }
+  t.nT = (int32_t)cdiv(T, t.L);
+  t.nBlk = (int32_t)(cols * t.nT);
+  return t;
+}
+
 // Restores the calling thread's current device on scope exit.
 struct DeviceGuard {
   int prev = -1;
@@ -676,6 +720,7 @@ struct BwdPlan {
   ReduceParams r{};
   bool skip = false;   // dim == 0: nothing to do
   bool empty = false;  // batch == 0 or seqlen == 0: the fill path
+  bool mfma = false;
   bool fast = false;
   bool wide = false;   // generic path above kMaxBlockW: g goes through the workspace
   int x_dt = 0;
@@ -687,6 +732,7 @@ struct BwdPlan {
 // kernels when the x dtype, the width and the alignment of every row of x, dout and dx (and of
 // dfinal_states) allow them, else the generic ones.
 struct BwdPath {
+  bool mfma = false;
   bool fast = false;
   bool wide = false;   // generic path above kMaxBlockW: g goes through the workspace
   Tiling tl{};
@@ -698,9 +744,19 @@ struct BwdPath {
 BwdPath bwd_path(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype, bool seq,
                  const void* dout, int64_t dout_stride_b, int64_t dout_stride_t,
                  const void* dfinal_states, const void* dx, int64_t dx_stride_b,
-                 int64_t dx_stride_t, bool ws_aligned, int64_t B, int64_t T, int64_t D,
+                 int64_t dx_stride_t, bool ws_aligned, bool mfma, int64_t B, int64_t T, int64_t D,
                  int64_t W) {
   BwdPath r;
+  r.mfma = mfma && rows_ok(x_dtype, 2, T, D, x, x_stride_t) &&
+           rows_ok(x_dtype, 2, T, D, dout, dout_stride_t) &&
+           rows_ok(x_dtype, 2, T, D, dx, dx_stride_t) &&
+           (!dfinal_states || aligned_to(dfinal_states, esize(x_dtype))) && ws_aligned;
+  if (r.mfma) {
+    r.tl = mfma_tiling(B, T, D, W);
+    r.rows = B * r.tl.nT;
+    r.need = partial_bytes(r.rows, W, D);
+    return r;
+  }
   const int bcpl = bwd_shape(x_dtype, B, T, D, W).cpl;
   r.fast = fast_dtype(x_dtype, W) && rows_ok(x_dtype, bcpl, T, D, x, x_stride_t) &&
            rows_ok(x_dtype, bcpl, T, D, dout, dout_stride_t) &&
@@ -809,14 +865,22 @@ int plan_bwd(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype,
 
   const BwdPath path = bwd_path(x, x_stride_b, x_stride_t, x_dtype, seq_idx != nullptr, dout,
                                 dout_stride_b, dout_stride_t, dfinal_states, dx, dx_stride_b,
-                                dx_stride_t, ws_aligned, B, T, D, W);
+                                dx_stride_t, ws_aligned,
+                                mfma_takes(x_dtype, D, W, silu != 0, seq_idx != nullptr,
+                                           initial_states != nullptr, init_dtype),
+                                B, T, D, W);
+  pl.mfma = path.mfma;
   pl.fast = path.fast;
   pl.wide = path.wide;
   p.tl = path.tl;
-  if (pl.fast) {
+  if (pl.mfma || pl.fast) {
     p.x_bytes = slab_bytes(x_dtype, T, D, x_stride_t);
     p.y_bytes = slab_bytes(x_dtype, T, D, dout_stride_t);
     p.o_bytes = slab_bytes(x_dtype, T, D, dx_stride_t);
+  }
+  if (pl.mfma) {
+    // nothing else to choose
+  } else if (pl.fast) {
     const int es = esize(x_dtype);
     p.tl.col_fast = W <= kColFastMaxW &&
                     (rows_off(dx, dx_stride_b, dx_stride_t, B, T, es, 128) ||
@@ -861,7 +925,9 @@ int run_bwd(BwdPlan& pl, void* workspace, int device, void* stream, bool timed) 
   hipError_t e;
   {
     const TimedLaunch timing(timed);
-    if (pl.fast) {
+    if (pl.mfma) {
+      e = launch_bwd_mfma(p, s);
+    } else if (pl.fast) {
       switch (pl.x_dt) {
         case CCV1D_BF16: e = launch_bwd_fast_t<__bf16>(p, s); break;
         case CCV1D_F16: e = launch_bwd_fast_t<_Float16>(p, s); break;
@@ -902,10 +968,15 @@ size_t ccv1d_bwd_workspace_bytes_for(const void* x, int64_t x_stride_b, int64_t 
   const int64_t B = batch, T = seqlen, D = dim, W = width;
   if (B <= 0 || T <= 0 || D <= 0 || W < 2 || !valid_dt(x_dtype)) return 0;
   if (x_stride_b < 0 || x_stride_t < 0 || dout_stride_b < 0 || dout_stride_t < 0) return 0;
-  const size_t need = bwd_path(x, x_stride_b, x_stride_t, x_dtype, seq_idx != nullptr, dout,
-                               dout_stride_b, dout_stride_t, dfinal_states, dx, T * D, D, true, B,
-                               T, D, W)
-                          .need;
+  // The activation and the initial states' dtype, which the query does not know, decide between the
+  // matrix cores and the vector kernels: the larger of their needs.
+  size_t need = 0;
+  for (const bool mfma : {false, mfma_takes(x_dtype, D, W, true, seq_idx != nullptr, false, 0)}) {
+    const BwdPath path =
+        bwd_path(x, x_stride_b, x_stride_t, x_dtype, seq_idx != nullptr, dout, dout_stride_b,
+                 dout_stride_t, dfinal_states, dx, T * D, D, true, mfma, B, T, D, W);
+    if (path.need > need) need = path.need;
+  }
   // Rows that do not start on the lanes' access width may be given to either family of kernels:
   // the larger of their needs.
   const int cpl = fast_dtype(x_dtype, W) ? bwd_shape(x_dtype, B, T, D, W).cpl : 1;

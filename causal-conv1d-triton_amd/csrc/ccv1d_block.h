@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kBlkNW * 64, 2) void fwd_block_kernel(const FwdPara
     int own = slot + NC;
     own = own >= NB ? own - NB : own;
     put(own, r0, nxt);
-    __syncthreads();
+    lds_barrier();
     if (a + kBlkStep < t1) rows.load(r0 + kBlkStep, nxt);
     float z[kBlk];
     // Rows of one sequence (the window's included): every mask is 1.
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(kBlkNW * 64, 2) void fwd_block_kernel(const FwdPara
       if (p.silu) v = v * sigmoid_f(v);
       if (active && r0 + r < t1) ob[(int64_t)(r0 + r) * D] = to_store<TX>(v);
     }
-    __syncthreads();  // the step's oldest blocks are overwritten next
+    lds_barrier();  // the step's oldest blocks are overwritten next
     slot += kBlkNW;
     slot = slot >= NB ? slot - NB : slot;
   }
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(kBlkNW * 64, 2) void bwd_block_kernel(const BwdPara
       cy[r] = ny[r];
     }
     put(own, r0, cx);
-    __syncthreads();
+    lds_barrier();
     if (a + kBlkStep - Pp < own_end) load(r0 + kBlkStep);
 
     float g[kBlk];
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(kBlkNW * 64, 2) void bwd_block_kernel(const BwdPara
 #pragma unroll
       for (int r = 0; r < kBlk; ++r) q[r * 64] = g[r];
     }
-    __syncthreads();
+    lds_barrier();
 
     // dx of the rows Pp before this wave's.
     const int u0 = r0 - Pp;
@@ -484,7 +484,7 @@ __global__ __launch_bounds__(kBlkNW * 64, 2) void bwd_block_kernel(const BwdPara
         for (int q = 0; q < kBlk; ++q) dw[n][q] += acc[q];
       }
     }
-    __syncthreads();  // the step's oldest blocks are overwritten next
+    lds_barrier();  // the step's oldest blocks are overwritten next
     base += kBlkNW;
     base = base >= NB ? base - NB : base;
   }
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(kBlkNW * 64, 2) void bwd_block_kernel(const BwdPara
   // the g ring after them, is free now).
   wl[wave * 64 + lane] = dwp;
   wl[(kBlkNW + wave) * 64 + lane] = db;
-  __syncthreads();
+  lds_barrier();
   float* pp = p.part + ((int64_t)b * p.tl.nT + tile) * (W + 1) * D + c;
   if (!active) return;
   const int sh = Pp - P;

@@ -1,0 +1,31 @@
+// Launcher of the matrix-core backward (bf16 x, silu, no seq_idx).
+#include "ccv1d_launch.h"
+#include "ccv1d_mfma.h"
+
+namespace ccv1d {
+
+template <int NC>
+static hipError_t mfma_nc(const BwdParams& p, hipStream_t s) {
+  static std::atomic<uint64_t> lds_allowed{0};
+  constexpr size_t shmem = MmShape<NC>::BYTES;
+  static_assert(shmem <= 160 * 1024, "LDS of one gfx950 CU");
+  const void* k = reinterpret_cast<const void*>(&bwd_mfma_kernel<NC>);
+  const hipError_t e = allow_lds(k, shmem, shmem, lds_allowed);
+  if (e != hipSuccess) return e;
+  return launch(k, dim3((unsigned)p.tl.nBlk), dim3(kMmNW * 64), shmem, s, &p);
+}
+
+hipError_t launch_bwd_mfma(const BwdParams& p, hipStream_t s) {
+  switch ((p.W - 1 + 15) / 16) {
+    case 2: return mfma_nc<2>(p, s);
+    case 3: return mfma_nc<3>(p, s);
+    case 4: return mfma_nc<4>(p, s);
+    case 5: return mfma_nc<5>(p, s);
+    case 6: return mfma_nc<6>(p, s);
+    case 7: return mfma_nc<7>(p, s);
+    case 8: return mfma_nc<8>(p, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace ccv1d

@@ -406,10 +406,22 @@ __device__ __forceinline__ int32_t seq_at(const int32_t* seqb, int t, int T, boo
   return seqb[t];
 }
 
+// Barrier for data exchanged through LDS only: waits for this wave's LDS operations, not for its
+// global loads, so prefetches stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Widths up to kMaxBlockW without a vectorised instance take the block kernels (ccv1d_block.h), whose
 // segments are whole steps of kBlkStep rows.
 constexpr int kMaxBlockW = 128;
 constexpr int kBlkStep = 64;
+
+// The matrix-core backward (ccv1d_mfma.h) works on 32 channels and steps of 256 rows.
+constexpr int kMmCh = 32;
+constexpr int kMmRows = 256;
 
 // Maps the hardware workgroup id to a logical one so that each of the 8 XCDs (which receive
 // workgroups round-robin) runs one contiguous range of logical workgroups. Neighbouring time tiles,

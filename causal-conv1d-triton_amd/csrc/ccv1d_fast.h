@@ -623,14 +623,6 @@ struct BwdLane {
   }
 };
 
-// Barrier for data exchanged through LDS only: waits for this wave's LDS operations, not for its
-// global loads, so prefetches stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // Waves per SIMD the backward's register budget is sized for: 4 (at most 128 VGPRs) up to width 4
 // and at width 5 with rows of at most 8 bytes (there the fp16 instance with seq_idx spills 16
 // bytes per lane); otherwise 2 (at most 256), within which the instances' own allocation sets the

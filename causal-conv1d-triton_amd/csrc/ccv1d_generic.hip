@@ -1,31 +1,11 @@
 // Launchers of the block kernels (widths up to 128), the scalar kernels (any width), the partial-sum
 // reduction and the fill kernel.
-#include <atomic>
-
 #include "ccv1d_block.h"
 #include "ccv1d_launch.h"
 
 namespace ccv1d {
 
 static_assert(blk_lds_bytes(kMaxBlockW, 4, true) <= 160 * 1024, "LDS of one gfx950 CU");
-
-// Dynamic LDS above the default 64 KiB per workgroup must be allowed per kernel first. Each block
-// kernel is allowed the most any width takes (at most the 160 KiB of a gfx950 CU) once per device, on
-// its first launch there that needs more than 64 KiB: later launches, including those recorded into
-// a captured graph, make no runtime call for it. `done` is the kernel's own set of devices (bit d for
-// device d < 64; others set it every launch).
-static hipError_t allow_lds(const void* kernel, size_t bytes, size_t max_bytes,
-                            std::atomic<uint64_t>& done) {
-  if (bytes <= 65536) return hipSuccess;
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
-  if (bit && (done.load(std::memory_order_acquire) & bit)) return hipSuccess;
-  e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_bytes);
-  if (e == hipSuccess && bit) done.fetch_or(bit, std::memory_order_acq_rel);
-  return e;
-}
 
 // Whether the x ring holds TX itself: 16-bit x, with initial states (if any) of the same type.
 template <typename TX, typename Params>

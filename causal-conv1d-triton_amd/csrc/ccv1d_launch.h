@@ -6,6 +6,8 @@
 
 #include <hip/hip_ext.h>
 
+#include <atomic>
+
 #include "ccv1d_device.h"
 
 namespace ccv1d {
@@ -114,6 +116,24 @@ inline hipError_t launch(const void* kernel, dim3 grid, dim3 block, size_t shmem
   return launch_args(kernel, grid, block, shmem, s, args);
 }
 
+// Dynamic LDS above the default 64 KiB per workgroup must be allowed per kernel first. Each
+// kernel is allowed the most any width takes (at most the 160 KiB of a gfx950 CU) once per device, on
+// its first launch there that needs more than 64 KiB: later launches, including those recorded into
+// a captured graph, make no runtime call for it. `done` is the kernel's own set of devices (bit d for
+// device d < 64; others set it every launch).
+inline hipError_t allow_lds(const void* kernel, size_t bytes, size_t max_bytes,
+                            std::atomic<uint64_t>& done) {
+  if (bytes <= 65536) return hipSuccess;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
+  if (bit && (done.load(std::memory_order_acquire) & bit)) return hipSuccess;
+  e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_bytes);
+  if (e == hipSuccess && bit) done.fetch_or(bit, std::memory_order_acq_rel);
+  return e;
+}
+
 // The vectorised kernels are instantiated in translation units of their own per pass, dtype and
 // width range, so the build compiles them in parallel: widths 2..8 (ccv1d_{fwd,bwd}_<dtype>.hip),
 // 9..16 (_wide.hip), 17..24 (_long1.hip) and 25..32 (_long2.hip). First widths of the last three:
@@ -154,6 +174,8 @@ hipError_t launch_bwd_generic_t(const BwdParams& p, hipStream_t s);
 // the partial rows from it (the second is the main kernel for ccv1d_time_main_kernel).
 template <typename TX>
 hipError_t launch_bwd_wide_t(const BwdParams& p, float* G, hipStream_t s);
+// Matrix-core backward: bf16 x, silu, no seq_idx, dim >= 32, initial states of x's dtype.
+hipError_t launch_bwd_mfma(const BwdParams& p, hipStream_t s);
 hipError_t launch_reduce(const ReduceParams& p, hipStream_t s);
 hipError_t launch_fill(void* dst, int dst_dt, const void* src, int src_dt, int64_t n, hipStream_t s);
 

@@ -1394,3 +1394,47 @@ def test_block_kernel_long_segments(W, seq):
     gpu = run_gpu(inp, "silu", init_grad=True)
     cols = _cols(D, 6, W)
     compare(gpu, oracle_ref(inp, True, cols=cols, need_dinit=True), True, cols)
+
+
+@pytest.mark.parametrize("W", [33, 48, 64, 81, 100, 113, 128])
+def test_matrix_core_backward(W):
+    """bf16 x with silu from width 33: the backward on the matrix cores, one width for each count of
+    16-row window blocks. Lengths inside one step of 256 rows, around steps and windows, and (the
+    last shape) of several steps per segment; a dim that 32-channel blocks do not divide; states and
+    their gradients."""
+    for T, D in ((1, 33), (W, 32), (255, 40), (257, 65), (512 + W, 33)):
+        inp = make_inputs(31 * W + T, 2, T, D, W, bias=T % 2 == 1, init=D % 2 == 1)
+        gpu = run_gpu(inp, "silu", return_final=True, dfinal=True, init_grad=D % 2 == 1)
+        compare(gpu, oracle_ref(inp, True, final=True, dfinal=True, need_dinit=D % 2 == 1), True)
+    inp = make_inputs(37 * W, 4, 2900, 1100, W, init=True)
+    gpu = run_gpu(inp, "silu", init_grad=True)
+    cols = _cols(1100, 6, W)
+    compare(gpu, oracle_ref(inp, True, cols=cols, need_dinit=True), True, cols)
+
+
+@pytest.mark.parametrize("W", [33, 64, 120])
+def test_matrix_core_backward_keeps_non_finite_values_in_their_windows(W):
+    """An infinity or NaN in x, dout or the weights reaches exactly the gradients it reaches in the
+    oracle (the matrix products' zero entries do not spread it), and the other values stay right."""
+    B, T, D = 2, 900, 40
+    inp = make_inputs(41 * W, B, T, D, W, init=True)
+    inp["x"][0, 100, 3] = float("inf")
+    inp["x"][1, 254, 5] = float("nan")     # beside a step's edge
+    inp["x"][1, 500, 6] = 1e30
+    inp["dy"][0, 400, 7] = float("inf")
+    inp["dy"][1, 256, 9] = float("nan")
+    inp["w"][11, 2] = float("inf")
+    inp["init"][1, 4, 13] = float("nan")
+    gpu = run_gpu(inp, "silu", init_grad=True)
+    ref = oracle_ref(inp, True, need_dinit=True)
+    for k in ("out", "dx", "dinit", "dw", "db"):
+        r = torch.from_numpy(np.ascontiguousarray(ref[k]))
+        assert torch.equal(gpu[k].isnan(), r.isnan()), k
+        ok = r.isfinite() & (r.abs() < 1e30)
+        assert bool(gpu[k][ok].isfinite().all()), k
+        if k in ("dw", "db"):
+            keep = torch.ones(D, dtype=torch.bool)
+            keep[[3, 5, 6, 7, 9, 11, 13]] = False
+            check_sum(gpu[k][keep], ref[k][keep.numpy()], k)
+        else:
+            check_lowp(gpu[k][ok], r[ok].numpy(), False, k)
