@@ -356,20 +356,52 @@ size_t g_buffer_bytes(int64_t B, int64_t T, int64_t D) {
 }
 size_t g_buffer_offset(size_t partials) { return (partials + 255) & ~(size_t)255; }
 
+// Rows per segment for kernels whose workgroups each walk a segment of one of `cols` columns in steps:
+// all of them do about the same work, so what counts is how many of them one after the other a slot
+// of the chip runs (`slots` workgroups at once on 256 CUs) and what each costs. Of the segment
+// counts that just fill 1, 2, ... rounds, the cheapest; segments are multiples of `unit` rows and at
+// least `shortest`. cost(rows): a segment's cost in steps.
+template <typename Cost>
+int64_t fill_rounds(int64_t T, int64_t cols, int64_t slots, int64_t unit, int64_t shortest,
+                    const Cost& cost) {
+  constexpr int64_t kMaxRounds = 8;
+  int64_t best = -1, rows = shortest;
+  for (int64_t r = 1; r <= kMaxRounds; ++r) {
+    int64_t n = slots * r / cols;
+    n = n < 1 ? 1 : n;
+    int64_t L = cdiv(cdiv(T, n), unit) * unit;
+    const bool last = L <= shortest;
+    if (last) L = shortest;
+    const double c = (double)cdiv(cols * cdiv(T, L), slots) * cost(L);
+    if (best < 0 || c < (double)best / 16) {
+      best = (int64_t)(c * 16);
+      rows = L;
+    }
+    if (last) break;
+  }
+  return rows;
+}
+
 // Tiling of the kernels without compile-time widths. Above kMaxBlockW: tiles of kGenericL rows. Up
-// to it a workgroup of the block kernels walks a segment of whole steps, and each segment reads a
-// window of rows and the weights once more (the backward also forms g of a window past its end): the
-// longest segment that still gives the grid kBlkTargetGroups workgroups, 2 per CU. A segment is
-// never shorter than kGenericL rows, so there are never more partial rows than of kGenericL-row tiles.
-constexpr int64_t kBlkTargetGroups = 512;
-constexpr int kBlkMaxRows = 2048;
-static_assert(kGenericL % kBlkStep == 0, "segments are whole steps");
-Tiling generic_tiling(int64_t B, int64_t T, int64_t D, int64_t W) {
+// to it segments of the block kernels, whole steps: a CU holds as many workgroups as their LDS
+// allows, at most 4 in the forward and 2 in the backward (registers); the start (weights, window)
+// costs about a step and half a step per window, and the backward walks a window past its segment.
+// Forward alone B=2 T=4096 D=1024 bf16, power-of-two segments for 512 workgroups before: W=64 33.9
+// -> 30.3 us, W=33 25.6 -> 21.8; fwd+bwd fp32 W=64 197 -> 180, B=1 T=16384 D=512 107 -> 98.
+// Never more partial rows than of kGenericL-row tiles.
+Tiling generic_tiling(int64_t B, int64_t T, int64_t D, int64_t W, int x_dt, bool bwd) {
+  static_assert(kGenericL % kBlkStep == 0, "segments are whole steps");
   Tiling t{};
   t.L = kGenericL;
   if (W <= kMaxBlockW) {
-    t.L = kBlkMaxRows;
-    while (t.L > kGenericL && B * cdiv(D, 64) * cdiv(T, t.L) < kBlkTargetGroups) t.L /= 2;
+    const int xs = esize(x_dt) == 2 ? 2 : 4;
+    const int64_t fit = (160 << 10) / (int64_t)blk_lds_bytes((int)W, xs, bwd);
+    const int64_t most = bwd ? 2 : 4;
+    const int64_t window = blk_window((int)W);
+    t.L = (int32_t)fill_rounds(
+        T, B * cdiv(D, 64), 256 * (fit < most ? fit : most), kBlkStep, kGenericL, [&](int64_t L) {
+          return (double)cdiv(L + (bwd ? window : 0), kBlkStep) + 1.0 + 0.5 * window / kBlkStep;
+        });
   }
   t.nT = (int32_t)cdiv(T, t.L);
   return t;
@@ -384,38 +416,18 @@ bool mfma_takes(int x_dt, int64_t D, int64_t W, bool silu, bool seq, bool init, 
          (!init || i_dt == x_dt);
 }
 
-// Its tiling. Every workgroup does about the same work, so what counts is how many of them one after
-// the other a CU runs (256 CUs, one at a time) and how many steps each takes: a segment and its
-// window are walked in whole steps, and a workgroup's start and end (weights, sums) cost about one
-// more. Of the segment counts that just fill 1, 2, ... rounds, the cheapest: with the longest segments
-// of 8 steps that still filled the chip, rows left over ran a second round (B=2 T=4096 D=1024 W=64
-// 170 -> 115 us, B=4 T=8192 D=1024 W=32 292 -> 212).
-constexpr int kMmMaxRounds = 8;
+// Its tiling: one workgroup per CU at a time; a segment and its window are walked in whole steps, and
+// the start and end (weights, sums) cost about one more. (With the longest segments of 8 steps that
+// still filled the chip, rows left over ran a second round: B=2 T=4096 D=1024 W=64 170 -> 115 us.) Only
+// a row's first segment has a window outside x, so segments are at least a window long.
 Tiling mfma_tiling(int64_t B, int64_t T, int64_t D, int64_t W) {
   Tiling t{};
-  const int64_t window = cdiv(W - 1, 16) * 16;
-  constexpr int64_t slots = 256;
-  // Only a row's first segment has a window outside x, and never more partial rows than of
-  // kGenericL-row tiles.
-  const int64_t shortest = window < kGenericL ? kGenericL : window;
+  const int64_t window = blk_window((int)W);
   t.nGW = (int32_t)cdiv(D, kMmCh);
-  const int64_t cols = B * t.nGW;
-  int64_t best = -1;
-  for (int64_t r = 1; r <= kMmMaxRounds; ++r) {
-    int64_t n = slots * r / cols;
-    n = n < 1 ? 1 : n;
-    const int64_t L = cdiv(cdiv(T, n), 16) * 16;
-    if (L < shortest && best >= 0) break;
-    const int64_t Ls = L < shortest ? shortest : L;
-    const int64_t groups = cols * cdiv(T, Ls);
-    const int64_t cost = cdiv(groups, slots) * (cdiv(Ls + window, kMmRows) + 1);
-    if (best < 0 || cost < best) {
-      best = cost;
-      t.L = (int32_t)Ls;
-    }
-  }
+  t.L = (int32_t)fill_rounds(T, B * t.nGW, 256, 16, window < kGenericL ? kGenericL : window,
+                             [&](int64_t L) { return (double)cdiv(L + window, kMmRows) + 1.0; });
   t.nT = (int32_t)cdiv(T, t.L);
-  t.nBlk = (int32_t)(cols * t.nT);
+  t.nBlk = (int32_t)(B * t.nGW * t.nT);
   return t;
 }
 
@@ -568,7 +580,7 @@ int fwd_entry(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype
                     (rows_off(x, x_stride_b, x_stride_t, B, T, esize(x_dtype), 128) ||
                      rows_off(out, T * D, D, B, T, esize(x_dtype), 128));
     } else {
-      tl = generic_tiling(B, T, D, W);
+      tl = generic_tiling(B, T, D, W, x_dtype, false);
       if (B * tl.nT >= (int64_t(1) << 31) || cdiv(D, 64) > 65535)
         return fail(CCV1D_ERR_UNSUPPORTED, "shape too large for the generic kernel");
     }
@@ -766,7 +778,7 @@ BwdPath bwd_path(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dt
     r.tl = bwd_fast_tiling(B, T, D, W, x_dtype, seq);
     r.rows = B * r.tl.nTB;
   } else {
-    r.tl = generic_tiling(B, T, D, W);
+    r.tl = generic_tiling(B, T, D, W, x_dtype, true);
     r.rows = B * r.tl.nT;
     r.wide = W > kMaxBlockW;
   }

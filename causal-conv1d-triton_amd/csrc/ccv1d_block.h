@@ -12,7 +12,7 @@
 //
 // Measured against one lane walking one row at a time with weights, x, g and the dweight sums in LDS
 // (four LDS accesses per tap; the kernels these replaced): B=2 T=4096 D=1024 W=64 bf16 fwd+bwd 5012
-// -> 138 us, forward alone 657 -> 35; W=33 107 us, W=128 350.
+// -> 138 us, forward alone 657 -> 36; with the segments of generic_tiling 30.
 //
 // Rows are numbered in taps of the padded window: with Pp = W - 1 rounded up to whole blocks, tap
 // k sits at position k + (Pp - P), so that every block of 16 positions meets whole row blocks. The
@@ -23,18 +23,6 @@
 #include "ccv1d_generic.h"
 
 namespace ccv1d {
-
-constexpr int kBlk = 16;
-constexpr int kBlkNW = 4;
-static_assert(kBlkStep == kBlk * kBlkNW, "a step is 16 rows per wave");
-constexpr int kBlkWPitch = 65;  // floats per weight row in LDS (64 channels; odd, see stage_weights)
-
-__host__ __device__ constexpr int blk_window(int W) { return (W - 1 + kBlk - 1) / kBlk * kBlk; }
-__host__ __device__ constexpr int blk_ring(int W) { return blk_window(W) / kBlk + kBlkNW; }
-// LDS bytes: weights, x ring (elements of xs bytes), g ring (backward), the rows' sequence ids.
-__host__ __device__ constexpr size_t blk_lds_bytes(int W, int xs, bool bwd) {
-  return (size_t)W * kBlkWPitch * 4 + (size_t)blk_ring(W) * kBlk * (64 * (xs + (bwd ? 4 : 0)) + 4);
-}
 
 // 16 rows of one channel from a ring of NB blocks, the `i`-th block from slot `slot`.
 template <typename E>
@@ -135,13 +123,39 @@ __device__ __forceinline__ bool ring_one_id(const int32_t* sid, int NB, int slot
 // The weights of 64 channels from c0 in LDS, tap k of channel c at [k][c - c0]. The 64 * W weights
 // are read in memory order, so neighbouring threads write different taps of one channel: with 65
 // floats per tap they meet different banks.
+// A thread requests 8 of them at a time (one load and its use at a time cost a memory round trip each,
+// 16 of them at W = 64: forward alone B=2 T=4096 D=1024 W=64 36.2
+// -> 33.9 us).
 __device__ __forceinline__ void stage_weights(const void* w, int w_dt, int c0, int D, int W,
                                               float* wl) {
+  constexpr int N = 8, NT = kBlkNW * 64;
   const int n = min(64, D - c0) * W;
-  const int64_t base = (int64_t)c0 * W;
-  for (int i = threadIdx.x; i < n; i += kBlkNW * 64) {
-    const int c = i / W;
-    wl[(i - c * W) * kBlkWPitch + c] = ld_any(w, base + i, w_dt);
+  const int dc = NT / W, dk = NT - dc * W;  // NT weights further on: dc channels and dk taps
+  int c = threadIdx.x / W, k = threadIdx.x - c * W;
+  auto each = [&](auto* q) {
+    q += (int64_t)c0 * W;
+#pragma unroll 1
+    for (int i = threadIdx.x; i < n; i += N * NT) {
+      float v[N];
+#pragma unroll
+      for (int u = 0; u < N; ++u) v[u] = static_cast<float>(q[min(i + u * NT, n - 1)]);
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        if (i + u * NT < n) wl[k * kBlkWPitch + c] = v[u];
+        k += dk;
+        c += dc;
+        if (k >= W) {
+          k -= W;
+          ++c;
+        }
+      }
+    }
+  };
+  switch (w_dt) {
+    case DT_F32: each(static_cast<const float*>(w)); break;
+    case DT_F16: each(static_cast<const _Float16*>(w)); break;
+    case DT_BF16: each(static_cast<const __bf16*>(w)); break;
+    default: each(static_cast<const double*>(w)); break;
   }
 }
 

@@ -417,7 +417,17 @@ __device__ __forceinline__ void lds_barrier() {
 // Widths up to kMaxBlockW without a vectorised instance take the block kernels (ccv1d_block.h), whose
 // segments are whole steps of kBlkStep rows.
 constexpr int kMaxBlockW = 128;
-constexpr int kBlkStep = 64;
+constexpr int kBlk = 16;
+constexpr int kBlkNW = 4;                  // waves per workgroup, 16 rows each per step
+constexpr int kBlkStep = kBlk * kBlkNW;
+constexpr int kBlkWPitch = 65;  // floats per weight row in LDS (64 channels; odd, see stage_weights)
+
+__host__ __device__ constexpr int blk_window(int W) { return (W - 1 + kBlk - 1) / kBlk * kBlk; }
+__host__ __device__ constexpr int blk_ring(int W) { return blk_window(W) / kBlk + kBlkNW; }
+// LDS bytes: weights, x ring (elements of xs bytes), g ring (backward), the rows' sequence ids.
+__host__ __device__ constexpr size_t blk_lds_bytes(int W, int xs, bool bwd) {
+  return (size_t)W * kBlkWPitch * 4 + (size_t)blk_ring(W) * kBlk * (64 * (xs + (bwd ? 4 : 0)) + 4);
+}
 
 // The matrix-core backward (ccv1d_mfma.h) works on 32 channels and steps of 256 rows.
 constexpr int kMmCh = 32;
