@@ -407,7 +407,7 @@ Tiling generic_tiling(int64_t B, int64_t T, int64_t D, int64_t W, int x_dt, bool
   return t;
 }
 
-// The matrix-core backward (ccv1d_mfma.h): bf16 x with silu, without seq_idx, and initial states (if
+// The matrix-core kernels (ccv1d_mfma.h, ccv1d_mfma_fwd.h): bf16 x with silu, without seq_idx, and initial states (if
 // any) of x's dtype. Without an activation the vector kernels stay: their results are the reference's
 // operation order bit for bit.
 constexpr int64_t kMmMinW = kMaxFastW + 1;  // see ccv1d_mfma.h
@@ -426,6 +426,23 @@ Tiling mfma_tiling(int64_t B, int64_t T, int64_t D, int64_t W) {
   t.nGW = (int32_t)cdiv(D, kMmCh);
   t.L = (int32_t)fill_rounds(T, B * t.nGW, 256, 16, window < kGenericL ? kGenericL : window,
                              [&](int64_t L) { return (double)cdiv(L + window, kMmRows) + 1.0; });
+  t.nT = (int32_t)cdiv(T, t.L);
+  t.nBlk = (int32_t)(B * t.nGW * t.nT);
+  return t;
+}
+
+// The forward's: two workgroups per CU (with as many as the LDS holds, 3 or 4, the shorter segments
+// they get cost more than the rounds saved: B=2 T=4096 D=1024 W=64 16.6 -> 21.1 us); segments above
+// 256 rows take steps of 512, which share the weights' fragments (16.6 -> 15.0 us) and cost 1.75
+// steps of 256; the start costs about one.
+Tiling mfma_fwd_tiling(int64_t B, int64_t T, int64_t D, int64_t W) {
+  Tiling t{};
+  const int64_t window = blk_window((int)W);
+  t.nGW = (int32_t)cdiv(D, kMmCh);
+  t.L = (int32_t)fill_rounds(T, B * t.nGW, 512, 16, window < kGenericL ? kGenericL : window,
+                             [&](int64_t L) {
+                               return 1.0 + (L > kMmRows ? 1.75 * (double)cdiv(L, 2 * kMmRows) : 1.0);
+                             });
   t.nT = (int32_t)cdiv(T, t.L);
   t.nBlk = (int32_t)(B * t.nGW * t.nT);
   return t;
@@ -572,9 +589,17 @@ int fwd_entry(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype
                     rows_ok(x_dtype, fcpl, T, D, x, x_stride_t) &&
                     rows_ok(x_dtype, fcpl, T, D, out, D) &&
                     (!final_states || aligned_to(final_states, esize(x_dtype)));
+  const bool mfma = T > 0 &&
+                    mfma_takes(x_dtype, D, W, silu != 0, seq_idx != nullptr,
+                               initial_states != nullptr, init_dtype) &&
+                    rows_ok(x_dtype, 2, T, D, x, x_stride_t) && rows_ok(x_dtype, 2, T, D, out, D) &&
+                    (!final_states || aligned_to(final_states, esize(x_dtype))) &&
+                    B * cdiv(D, kMmCh) * cdiv(T, kGenericL) < (int64_t(1) << 31);
   Tiling tl{};
   if (T > 0) {
-    if (fast) {
+    if (mfma) {
+      tl = mfma_fwd_tiling(B, T, D, W);
+    } else if (fast) {
       tl = fwd_fast_tiling(B, T, D, W, x_dtype, seq_idx != nullptr);
       tl.col_fast = W <= kColFastMaxW &&
                     (rows_off(x, x_stride_b, x_stride_t, B, T, esize(x_dtype), 128) ||
@@ -621,7 +646,7 @@ int fwd_entry(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype
   p.silu = silu != 0;
   p.out_nt = fwd_out_streams(inference, B, T, D, x_dtype);
   p.x_nt = tune().fwd_x_nt >= 0 ? tune().fwd_x_nt != 0 : inference && p.out_nt;
-  if (fast) {
+  if (mfma || fast) {
     p.x_bytes = slab_bytes(x_dtype, T, D, x_stride_t);
     p.o_bytes = slab_bytes(x_dtype, T, D, D);
   }
@@ -630,7 +655,9 @@ int fwd_entry(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype
   hipError_t e;
   {
     const TimedLaunch timing(timed);
-    if (fast) {
+    if (mfma) {
+      e = launch_fwd_mfma(p, s);
+    } else if (fast) {
       switch (x_dtype) {
         case CCV1D_BF16: e = launch_fwd_fast_t<__bf16>(p, s); break;
         case CCV1D_F16: e = launch_fwd_fast_t<_Float16>(p, s); break;

@@ -429,7 +429,8 @@ __host__ __device__ constexpr size_t blk_lds_bytes(int W, int xs, bool bwd) {
   return (size_t)W * kBlkWPitch * 4 + (size_t)blk_ring(W) * kBlk * (64 * (xs + (bwd ? 4 : 0)) + 4);
 }
 
-// The matrix-core backward (ccv1d_mfma.h) works on 32 channels and steps of 256 rows.
+// The matrix-core kernels (ccv1d_mfma.h, ccv1d_mfma_fwd.h) work on 32 channels, in steps of 256 rows
+// (the forward's segments above 256 rows: 512).
 constexpr int kMmCh = 32;
 constexpr int kMmRows = 256;
 

@@ -174,7 +174,8 @@ hipError_t launch_bwd_generic_t(const BwdParams& p, hipStream_t s);
 // the partial rows from it (the second is the main kernel for ccv1d_time_main_kernel).
 template <typename TX>
 hipError_t launch_bwd_wide_t(const BwdParams& p, float* G, hipStream_t s);
-// Matrix-core backward: bf16 x, silu, no seq_idx, dim >= 32, initial states of x's dtype.
+// Matrix-core kernels: bf16 x, silu, no seq_idx, dim >= 32, initial states of x's dtype.
+hipError_t launch_fwd_mfma(const FwdParams& p, hipStream_t s);
 hipError_t launch_bwd_mfma(const BwdParams& p, hipStream_t s);
 hipError_t launch_reduce(const ReduceParams& p, hipStream_t s);
 hipError_t launch_fill(void* dst, int dst_dt, const void* src, int src_dt, int64_t n, hipStream_t s);

@@ -1412,6 +1412,34 @@ def test_matrix_core_backward(W):
     compare(gpu, oracle_ref(inp, True, cols=cols, need_dinit=True), True, cols)
 
 
+@pytest.mark.parametrize("W", [33, 49, 64, 81, 112, 113, 128])
+@pytest.mark.parametrize("T", [257, 513, 1030])
+def test_matrix_core_forward_steps(W, T):
+    """The matrix-core forward in steps of 512 rows (a grid of as many channel blocks as the chip runs
+    at once has one segment per row), x a slice at an odd channel, around halves and ends of steps,
+    with infinities and NaN beside them: `out` and the final states."""
+    B, D = 8, 2047
+    inp = make_inputs(43 * W + T, B, T, D, W, init=True)
+    cols = _cols(D, 6, W)
+    c = int(cols[2])
+    for b, t in ((0, 255), (1, 256), (2, T - 1)):
+        inp["x"][b, t, c] = (float("inf"), float("nan"), float("-inf"))[b]
+    inp["w"][int(cols[3]), 1] = 3.4e38  # finite, and its first 8 bits rounded up are not
+    wide = torch.zeros(B, T, D + 9, dtype=inp["x"].dtype, device=DEV)
+    wide[..., 3:3 + D] = inp["x"].to(DEV)
+    out, fin = causal_conv1d_fn(wide[..., 3:3 + D], inp["w"].to(DEV), inp["b"].to(DEV),
+                                initial_states=inp["init"].to(DEV), return_final_states=True,
+                                activation="silu")
+    ref = oracle_ref(inp, True, cols=cols, bwd=False)
+    o, r = out.cpu()[..., cols], torch.from_numpy(np.ascontiguousarray(ref["out"]))
+    assert torch.equal(o.isnan(), r.isnan())
+    ok = r.isfinite() & (r.abs() < 1e30)
+    assert bool(o[ok].isfinite().all())
+    check_lowp(o[ok], r[ok].numpy(), False, "out")
+    want = torch.cat([inp["init"], inp["x"]], 1)[:, T:]
+    assert torch.equal(fin.cpu().view(torch.int16), want.contiguous().view(torch.int16))
+
+
 @pytest.mark.parametrize("W", [33, 64, 120])
 def test_matrix_core_backward_keeps_non_finite_values_in_their_windows(W):
     """An infinity or NaN in x, dout or the weights reaches exactly the gradients it reaches in the
