@@ -23,7 +23,11 @@
 // transposing read. A wave takes 4 of the channels. dx is written PP rows behind the rows of a step.
 //
 // Measured, fwd+bwd B=2 T=4096 D=1024 against the block kernels (ccv1d_block.h) in the backward:
-// W=33 107 -> 85 us, W=64 139 -> 108, W=100 306 -> 138, W=128 351 -> 158. What bounds it is the vector
+// W=33 107 -> 85 us, W=64 139 -> 108, W=100 306 -> 138, W=128 351 -> 158; then, with segments that fill
+// rounds and the matrix-core forward at 68.5, 85.7, 107.6 and 121.7, the weights' fragments kept from z
+// to dx (64.9, 82.2, 101.7) and no dweight products in a segment's last step where that holds dx rows
+// alone (63.7, 80.5, 98.7, 119.1; leaving z out there too past the end of x: T=256 W=40 121.4 -> 118.2, but
+// W=33 63.7 -> 64.4). What bounds it is the vector
 // work around the products (silu', the pieces, addresses: about 200 instructions per 256 elements)
 // at one workgroup per CU (the dweight tiles' registers); at widths 9-32 the register-window kernels
 // are faster (B=4 T=8192 D=1024 W=16 95 us against 150, W=32 159 against 210).
@@ -201,6 +205,7 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
   const int t0 = tile * p.tl.L;
   const int own_end = min(t0 + p.tl.L, T);
   const int emit_lo = (tile == 0 && p.need_dinit) ? -P : t0;
+  const int need_end = min(own_end + PP, T);
   const int steps = (own_end - t0 + PP + kMmRows - 1) / kMmRows;
 
   // Staging: a thread takes 8 rows of 2 channels.
@@ -223,7 +228,7 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
     asm volatile("" : "+v"(tid_));
     const int r0 = a + 8 * (tid_ >> 4);
     const uint32_t coff = (uint32_t)(c0 + 2 * (tid_ & 15)) * 2u;
-    if (a + kMmRows <= T) {
+    if (a + kMmRows <= need_end) {
       const uint32_t xo = (uint32_t)r0 * xrow + coff, yo = (uint32_t)r0 * yrow + coff;
 #pragma unroll
       for (int e = 0; e < 8; ++e)
@@ -231,10 +236,10 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         ry[e] = __builtin_amdgcn_raw_buffer_load_b32(yrs, yo, e * yrow, kCacheNT);
-    } else {  // rows past the end repeat the last one; their g is 0
+    } else {  // rows past the last one needed repeat it; past T their g is 0
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const uint32_t r = (uint32_t)min(r0 + e, T - 1);
+        const uint32_t r = (uint32_t)min(r0 + e, need_end - 1);
         rx[e] = __builtin_amdgcn_raw_buffer_load_b32(xrs, r * xrow + coff, 0, kCacheNT);
         ry[e] = __builtin_amdgcn_raw_buffer_load_b32(yrs, r * yrow + coff, 0, kCacheNT);
       }
@@ -389,7 +394,7 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
       const uint32_t* const wc = reinterpret_cast<const uint32_t*>(
           wp + ch * 3 * S::WL + ((8 * lq - li + 15) & ~1));
       const uint32_t wshift = (li & 1) ? 0 : 16;
-      auto weights = [&](int kb, int j) {
+      auto weights_at = [&](int kb, int j) {
         const uint32_t* q = wc + j * (S::WL / 2) + 16 * kb;
         uint32_t d[5];
 #pragma unroll
@@ -398,6 +403,19 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
 #pragma unroll
         for (int e = 0; e < 4; ++e) f[e] = __builtin_amdgcn_alignbit(d[e + 1], d[e], wshift);
         return __builtin_bit_cast(bf8v, f);
+      };
+      // Kept from z to dx up to 7 window blocks (at 8 they spill: W=128 121.7 -> 125.5 us).
+      constexpr bool kKeepW = NC <= 7;
+      bf8v wf[KB][3];
+      if constexpr (kKeepW) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) wf[kb][j] = weights_at(kb, j);
+      }
+      auto weights = [&](int kb, int j) {
+        if constexpr (kKeepW) return wf[kb][j];
+        else return weights_at(kb, j);
       };
       float gv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       u32x2 hi = {0u, 0u}, mid = {0u, 0u}, lo = {0u, 0u};
@@ -447,37 +465,39 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
           hi = mid = lo = u32x2{0u, 0u};
         }
       }
-      if (own < kMmRows) {  // rows past the segment count in dx only
+      if (own > 0) {  // else a step of dx rows alone (the segment's window)
+        if (own < kMmRows) {  // rows past the segment count in dx only
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const bool in = 64 * lq + 16 * v + li < own;
-          const uint32_t keep = in ? 0xffffffffu : (v & 1) ? 0x0000ffffu : 0xffff0000u;
-          hi[v >> 1] &= keep;
-          mid[v >> 1] &= keep;
-          lo[v >> 1] &= keep;
-          gv[v] = in ? gv[v] : 0.0f;
+          for (int v = 0; v < 4; ++v) {
+            const bool in = 64 * lq + 16 * v + li < own;
+            const uint32_t keep = in ? 0xffffffffu : (v & 1) ? 0x0000ffffu : 0xffff0000u;
+            hi[v >> 1] &= keep;
+            mid[v >> 1] &= keep;
+            lo[v >> 1] &= keep;
+            gv[v] = in ? gv[v] : 0.0f;
+          }
         }
-      }
-      db[n] += (gv[0] + gv[1]) + (gv[2] + gv[3]);
-      // K slots of a lane: rows b = 4 lq + v once with the first piece and once with the second.
-      const bf8v ga = __builtin_bit_cast(bf8v, (u32x4){hi[0], hi[1], mid[0], mid[1]});
-      const bf8v gb = __builtin_bit_cast(bf8v, (u32x4){lo[0], lo[1], 0u, 0u});
+        db[n] += (gv[0] + gv[1]) + (gv[2] + gv[3]);
+        // K slots of a lane: rows b = 4 lq + v once with the first piece and once with the second.
+        const bf8v ga = __builtin_bit_cast(bf8v, (u32x4){hi[0], hi[1], mid[0], mid[1]});
+        const bf8v gb = __builtin_bit_cast(bf8v, (u32x4){lo[0], lo[1], 0u, 0u});
 #pragma unroll
-      for (int m = 0; m <= NC; ++m) {
-        const u32x2 xv = mm_column(xc + 16 * (NC - m), ln);
-        const uint32_t x0 = fast ? xv[0] ^ flip : 0u, x1 = fast ? xv[1] ^ flip : 0u;
-        const bf8v xb = __builtin_bit_cast(bf8v, (u32x4){x0, x1, x0, x1});
-        // A step's products are summed from zero and the steps by vector adds. The matrix cores' sums
-        // are biased downwards by about 1 % of an ulp, which grows with the number of rows where
-        // the rounding errors themselves average out: every other step takes x negated.
-        f4v t = {0.0f, 0.0f, 0.0f, 0.0f};
-        t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gb, xb, t, 0, 0, 0);
-        t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga, xb, t, 0, 0, 0);
+        for (int m = 0; m <= NC; ++m) {
+          const u32x2 xv = mm_column(xc + 16 * (NC - m), ln);
+          const uint32_t x0 = fast ? xv[0] ^ flip : 0u, x1 = fast ? xv[1] ^ flip : 0u;
+          const bf8v xb = __builtin_bit_cast(bf8v, (u32x4){x0, x1, x0, x1});
+          // A step's products are summed from zero and the steps by vector adds. The matrix cores'
+          // sums are biased downwards by about 1 % of an ulp, which grows with the number of rows
+          // where the rounding errors themselves average out: every other step takes x negated.
+          f4v t = {0.0f, 0.0f, 0.0f, 0.0f};
+          t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gb, xb, t, 0, 0, 0);
+          t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga, xb, t, 0, 0, 0);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          float sum = fmaf(sign, t[v], acc[n][m][v]);
-          asm volatile("" : "+v"(sum));  // added here: the adds would sink past dx, all tiles' t held
-          acc[n][m][v] = sum;
+          for (int v = 0; v < 4; ++v) {
+            float sum = fmaf(sign, t[v], acc[n][m][v]);
+            asm volatile("" : "+v"(sum));  // added here: the adds would sink past dx, all t held
+            acc[n][m][v] = sum;
+          }
         }
       }
       mm_fence();
