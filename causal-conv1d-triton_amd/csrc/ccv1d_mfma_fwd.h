@@ -4,7 +4,9 @@
 // A workgroup takes 32 channels and walks a segment of rows in steps of 256 or 512. Rows are
 // transposed in registers into per-channel LDS rows; a wave takes 4 of the channels and leaves out in x's place,
 // which the thread that staged those rows reads back, transposes and stores. The weights are the
-// products' left operand, so that a lane ends up with 4 consecutive rows (one 8-byte LDS write).
+// products' left operand, so that a lane ends up with 4 consecutive rows (one 8-byte LDS write). A
+// row's sum is grouped by its place in its block of 16 rows from the call's first row on (segments
+// are multiples of 16), whatever the segment: chunks cut elsewhere can differ in out's last bit.
 //
 // Measured, forward alone B=2 T=4096 D=1024 against fwd_block_kernel: W=33 21.8 -> 13.2 us, W=64
 // 30.3 -> 14.8, W=128 47 -> 18.4 (memory: about 6). What bounds it is LDS reads and vector work around
