@@ -15,7 +15,9 @@
 //
 // Zeros of the Toeplitz matrix meet rows outside an output's window, so an infinity or NaN there would
 // spread: a channel whose x, dout, weights or g in reach are not all finite is computed with vector
-// arithmetic in its window alone (mm_slow).
+// arithmetic in its window alone (mm_slow). Each channel goes by its own values, never by those of
+// the 31 it shares a workgroup with: its results do not depend on them, and the two workgroups that
+// share channels where 32 does not divide dim store the same bits.
 //
 // A workgroup takes 32 channels and walks a segment of rows in steps of 256. Rows are read channels
 // last, transposed in registers (8 rows x 2 channels per lane) and kept per channel in time order in
@@ -80,6 +82,35 @@ __device__ __forceinline__ uint32_t bf_pack(float a, float b) {
 }
 __device__ __forceinline__ bool finite_f(float v) {
   return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u;
+}
+
+// Sets of a workgroup's 32 channels: channel ch is bit ch / 2 of its half, the even channels in the
+// lower 16 bits, so that the channels of one wave (wave + n * kMmNW) are every fourth bit from
+// mm_bit(wave) on.
+__device__ __forceinline__ int mm_bit(int ch) { return (ch >> 1) + ((ch & 1) << 4); }
+__device__ __forceinline__ uint32_t mm_wave_bits(uint32_t set, int wave) {
+  return set >> mm_bit(wave);  // bit 4 n: channel wave + n * kMmNW
+}
+static_assert(kMmNW == 8 && kMmCh == 32, "every fourth bit of a half");
+
+// The wave's channels whose staged rows hold an infinity or NaN: a thread has rows of channels
+// 2 (lane % 16) and the one after it, `bad` says so of them in bits 15 and 31.
+__device__ __forceinline__ uint32_t mm_bad_rows(uint32_t bad) {
+  const uint64_t e = __ballot((bad & 0x8000u) != 0), o = __ballot((bad & 0x80000000u) != 0);
+  uint32_t lo = (uint32_t)e | (uint32_t)(e >> 32), hi = (uint32_t)o | (uint32_t)(o >> 32);
+  lo |= lo >> 16;
+  hi |= hi << 16;
+  return (lo & 0xffffu) | (hi & 0xffff0000u);
+}
+
+// Those whose weights do: 16 lanes have the taps of one of the wave's 4 channels.
+__device__ __forceinline__ uint32_t mm_bad_taps(bool bad, int wave) {
+  const uint64_t b = __ballot(bad);
+  uint32_t set = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if ((b >> (16 * q)) & 0xffffu) set |= 1u << mm_bit(4 * wave + q);
+  return set;
 }
 
 // v as three bf16 pieces (bits) whose sum is v; false if v or its first piece is not finite.
@@ -200,7 +231,8 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
   const int tile = rest % p.tl.nT;
   const int b = rest / p.tl.nT;
   // The last block of a dim that is not a multiple of 32 is its last 32 channels: it shares channels with
-  // the block before, and both store the same bits for them.
+  // the block before, and both store the same bits for them (a channel's arithmetic, the choice of
+  // mm_slow included, depends on its own values alone).
   const int c0 = min(cb * kMmCh, D - kMmCh);
   const int t0 = tile * p.tl.L;
   const int own_end = min(t0 + p.tl.L, T);
@@ -326,14 +358,15 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
     db[n] = 0.0f;
   }
 
-  bool slow_prev = false, slow_w = false;
+  const uint32_t bad_taps = mm_bad_taps(wbad, wave);
+  int slow_prev = 0;  // channels of mm_slow by the step before, whose last rows are the window
 #pragma unroll 1
   for (int s = 0; s < steps; ++s) {
     const int a = t0 + s * kMmRows;
     put(rx, xs, S::XP, PP, bad);
     put(ry, ys, S::YP, 0, bad);
-    const int mine = (__any((bad & 0x80008000u) != 0) ? 1 : 0) | (__any(wbad) ? 2 : 0);
-    if (lane == 0) flag[wave] = mine;
+    const uint32_t mine = mm_bad_rows(bad) | bad_taps;
+    if (lane == 0) flag[wave] = (int32_t)mine;
     bad = 0;
     lds_barrier();
     if (s + 1 < steps) load(a + kMmRows);
@@ -341,9 +374,8 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
 #pragma unroll
     for (int v = 0; v < kMmNW; ++v) f |= flag[v];
     f = __builtin_amdgcn_readfirstlane(f);
-    slow_w = slow_w || (f & 2);
-    const bool slow = slow_w || slow_prev || (f & 1);
-    slow_prev = f & 1;
+    const uint32_t slow = mm_wave_bits((uint32_t)(slow_prev | f), wave);
+    slow_prev = f;
     const int rows_t = T - a;      // rows of the step before T (may be <= 0)
     const int own = own_end - a;   // its own rows (may be <= 0: only dx rows are left)
     const int row0 = a - PP;       // row of the step's first dx
@@ -386,7 +418,7 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
       int ln = lane;
       asm volatile("" : "+s"(ch), "+v"(ln));
       const int li = ln & 15, lq = ln >> 4;
-      bool fast = !slow && !(gbad >> n & 1);
+      bool fast = !(slow >> (4 * n) & 1) && !(gbad >> n & 1);
       const uint16_t* const xc = xs + ch * S::XP;
       uint16_t* const yc = ys + ch * S::YP;
       // A lane's 8 weights start at any element: 5 aligned words, shifted by one element where the

@@ -5,7 +5,8 @@
 // transposed in registers into per-channel LDS rows; a wave takes 4 of the channels and leaves out in x's place,
 // which the thread that staged those rows reads back, transposes and stores. The weights are the
 // products' left operand, so that a lane ends up with 4 consecutive rows (one 8-byte LDS write). A
-// row's sum is grouped by its place in its block of 16 rows from the call's first row on (segments
+// channel with infinities or NaN in reach is computed row by row, by its own values alone as in the
+// backward. A row's sum is grouped by its place in its block of 16 rows from the call's first row on (segments
 // are multiples of 16), whatever the segment: chunks cut elsewhere can differ in out's last bit.
 //
 // Measured, forward alone B=2 T=4096 D=1024 against fwd_block_kernel: W=33 21.8 -> 13.2 us, W=64
@@ -167,13 +168,14 @@ __global__ __launch_bounds__(kMmNW * 64, 4) void fwd_mfma_kernel(const FwdParams
     }
   }
 
-  bool slow_prev = false, slow_w = false;
+  const uint32_t bad_taps = mm_bad_taps(wbad, wave);
+  int slow_prev = 0;  // channels computed row by row by the step before, whose last rows are the window
 #pragma unroll 1
   for (int a = t0; a < t1; a += ROWS) {
 #pragma unroll
     for (int h = 0; h < SUB; ++h) put(rx[h], PP + h * kMmRows);
-    const int mine = (__any((bad & 0x80008000u) != 0) ? 1 : 0) | (__any(wbad) ? 2 : 0);
-    if (lane == 0) flag[wave] = mine;
+    const uint32_t mine = mm_bad_rows(bad) | bad_taps;
+    if (lane == 0) flag[wave] = (int32_t)mine;
     bad = 0;
     lds_barrier();
     if (a + ROWS < t1) load(a + ROWS);
@@ -181,9 +183,8 @@ __global__ __launch_bounds__(kMmNW * 64, 4) void fwd_mfma_kernel(const FwdParams
 #pragma unroll
     for (int v = 0; v < kMmNW; ++v) f |= flag[v];
     f = __builtin_amdgcn_readfirstlane(f);
-    slow_w = slow_w || (f & 2);
-    const bool slow = slow_w || slow_prev || (f & 1);
-    slow_prev = f & 1;
+    const uint32_t slow = mm_wave_bits((uint32_t)(slow_prev | f), wave);
+    slow_prev = f;
 
 #pragma unroll
     for (int n = 0; n < kMmPerWave; ++n) {
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(kMmNW * 64, 4) void fwd_mfma_kernel(const FwdParams
       uint16_t* const xc = xs + ch * S::XP;
       const float bias = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(bias_v), ch));
       float o[SUB][4];
-      if (!slow) {
+      if (!(slow >> (4 * n) & 1)) {
         // 8 weights of a lane from any element on: aligned words, shifted where the start is odd.
         const uint32_t* const wq = reinterpret_cast<const uint32_t*>(
             wp + ch * 3 * S::WL + ((8 * lq - li + 15) & ~1));
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(kMmNW * 64, 4) void fwd_mfma_kernel(const FwdParams
 #pragma unroll
           for (int v = 0; v < 4; ++v) o[h][v] = z[h][v] * sigmoid_f(z[h][v]);
         }
-      } else {  // infinities or NaN in reach: every row in its own window alone
+      } else {  // infinities or NaN in the channel's reach: every row in its own window alone
         const uint16_t* const wq = wp + ch * 3 * S::WL + sh + 15;
 #pragma unroll
         for (int h = 0; h < SUB; ++h) {

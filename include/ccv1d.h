@@ -25,7 +25,10 @@
  *  - Return value: CCV1D_OK (0) or an error code; ccv1d_last_error() then describes the failure.
  *  - Reentrant and thread-safe; the only global state is the error string and the timing request of
  *    ccv1d_time_main_kernel (both thread-local). The library reads nothing from the environment:
- *    its tiling, and with it every summation order, is a function of the shape alone.
+ *    its tiling, and with it every summation order, is a function of the shape alone. (One exception,
+ *    at widths 33 to 128 with bf16 x and silu: in a channel that holds an infinity or NaN the order
+ *    also depends on where that channel's own values are not finite. No channel's results depend on
+ *    another channel's values.)
  */
 #ifndef CCV1D_H
 #define CCV1D_H
@@ -147,7 +150,8 @@ size_t ccv1d_bwd_workspace_bytes_for(const void* x, int64_t x_stride_b, int64_t 
  *  workspace         device buffer of at least ccv1d_bwd_workspace_bytes() bytes (256-byte aligned);
  *                    may be NULL when that size is 0
  *
- * dweight and dbias are deterministic: the summation order depends only on the shape.
+ * dweight and dbias are deterministic: the summation order depends only on the shape (and, as stated
+ * at the top, on the places of a channel's own infinities and NaN at widths 33 to 128).
  */
 int ccv1d_bwd(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype,
               const void* weight, int weight_dtype,

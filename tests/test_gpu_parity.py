@@ -1466,3 +1466,30 @@ def test_matrix_core_backward_keeps_non_finite_values_in_their_windows(W):
             check_sum(gpu[k][keep], ref[k][keep.numpy()], k)
         else:
             check_lowp(gpu[k][ok], r[ok].numpy(), False, k)
+
+
+@pytest.mark.parametrize("W,B,T,D,c", [(33, 2, 700, 64, 3), (33, 2, 700, 40, 3), (64, 2, 700, 65, 3),
+                                       (64, 4, 1030, 2017, 1984), (113, 2, 700, 40, 3)])
+def test_matrix_core_channels_do_not_see_each_other(W, B, T, D, c):
+    """An infinity or NaN in one channel leaves every bit of every other channel's results as it is
+    without it: the channels that share a workgroup with it (D = 64 too), and those that two workgroups
+    compute where 32 does not divide dim, only one of which holds the channel. The fourth shape has
+    segments of several steps."""
+    inp = make_inputs(47 * W + D, B, T, D, W, init=True)
+
+    def run(i):
+        return run_gpu(i, "silu", return_final=True, dfinal=True, init_grad=True)
+
+    clean = run(inp)
+    others = torch.arange(D) != c
+    for name, at, value in (("x", (0, 100, c), float("inf")), ("x", (B - 1, 300, c), float("nan")),
+                            ("dy", (0, T - 5, c), float("inf")), ("init", (1, 7, c), float("nan")),
+                            ("w", (c, 2), float("inf"))):
+        bad = dict(inp)
+        bad[name] = inp[name].clone()
+        bad[name][at] = value
+        got = run(bad)
+        for k in ("out", "dx", "dinit"):
+            assert torch.equal(got[k][..., others], clean[k][..., others]), (name, k)
+        for k in ("dw", "db"):
+            assert torch.equal(got[k][others], clean[k][others]), (name, k)
