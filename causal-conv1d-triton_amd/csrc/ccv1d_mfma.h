@@ -64,7 +64,8 @@ struct MmShape {
   static constexpr int FLAG = WP + kMmCh * 3 * WL;      // one word per wave
   static constexpr int SUM = FLAG + 2 * kMmNW;          // floats [32][SP]: sums of mm_slow (dbias last)
   static constexpr int SP = PP + 2;
-  static constexpr int BYTES = 2 * SUM + 4 * kMmCh * SP;
+  static constexpr int TAPS = SUM + 2 * kMmCh * SP;     // floats [32][SP]: weights of mm_slow (bias last)
+  static constexpr int BYTES = 2 * TAPS + 4 * kMmCh * SP;
   static_assert(XP >= PP + kMmRows && GP >= PP + kMmRows && FLAG % 8 == 0, "layout");
   static_assert((kMaxBlockW + 1) * kMmCh * 2 <= kMmCh * YP, "dweight sums reuse the dout rows");
   static_assert(16 * 17 * 2 <= 3 * GP, "one tile of dweight lags reuses a wave's g rows");
@@ -151,19 +152,17 @@ __device__ __forceinline__ u32x2 mm_column(const uint16_t* p, int lane) {
   return __builtin_bit_cast(u32x2, v);
 }
 
-// One channel of one step in its rows' own windows, with vector arithmetic: g of the step's rows (its
-// pieces to `g`, whose last PP rows hold the previous ones), dx to `yc`, the sums of dweight and
-// dbias added to `sum`. rows_t: rows of the step before T; own: its own rows.
+// One channel of one step in its rows' own windows, with vector arithmetic: g~ = -ln2 g of the step's
+// rows (its pieces to `g`, whose last PP rows hold the previous ones), dx to `yc`, the sums of dweight
+// and dbias added to `sum`. rows_t: rows of the step before T; own: its own rows. `taps` (the bias
+// last) and pre-activations are the unscaled ones: times log2(e) as in the products, those above
+// 2.36e38 would be infinite.
 template <int NC, typename DF>
 __device__ __forceinline__ void mm_slow(const uint16_t* xc, uint16_t* yc, uint16_t* g,
-                                        const uint16_t* wc, int W, float bias, int rows_t, int own,
-                                        int lane, float* sum, const DF& dfinal) {
+                                        const float* taps, int W, int rows_t, int own, int lane,
+                                        float* sum, const DF& dfinal) {
   using S = MmShape<NC>;
   const int P = W - 1, sh = S::PP - P;
-  auto tap = [&](int k) {
-    const uint16_t* q = wc + k + sh + 15;
-    return bf_one(q[0]) + (bf_one(q[S::WL]) + bf_one(q[2 * S::WL]));
-  };
   auto g_at = [&](int r) {  // row r of the window (0 .. PP + 255)
     const uint16_t* q = g + S::PP + kMmRows - 1 - r;
     return bf_one(q[0]) + (bf_one(q[S::GP]) + bf_one(q[2 * S::GP]));
@@ -171,9 +170,9 @@ __device__ __forceinline__ void mm_slow(const uint16_t* xc, uint16_t* yc, uint16
   float db = 0.0f;
 #pragma unroll 1
   for (int r = lane; r < kMmRows; r += 64) {
-    float z = bias;
-    for (int k = 0; k < W; ++k) z = fmaf(tap(k), bf_one(xc[r + sh + k]), z);
-    const float gv = r < rows_t ? dsilu_scaled(bf_one(yc[r]), z) : 0.0f;
+    float z = taps[P] * bf_one(xc[r + sh + P]);
+    for (int k = 0; k < P; ++k) z = fmaf(taps[k], bf_one(xc[r + sh + k]), z);
+    const float gv = r < rows_t ? -kLn2 * dsilu_times(bf_one(yc[r]), z + taps[W]) : 0.0f;
     uint16_t pc[3];
     split3(gv, pc);
 #pragma unroll
@@ -184,8 +183,8 @@ __device__ __forceinline__ void mm_slow(const uint16_t* xc, uint16_t* yc, uint16
 #pragma unroll 1
   for (int r = lane; r < kMmRows; r += 64) {
     float d = 0.0f;
-    for (int j = 0; j <= P; ++j) d = fmaf(tap(P - j), g_at(r + j), d);
-    d += dfinal(r);
+    for (int j = 0; j <= P; ++j) d = fmaf(taps[P - j], g_at(r + j), d);
+    d = fmaf(d, kNegLog2e, dfinal(r));
     yc[r] = (uint16_t)(bf_pack(d, 0.0f) & 0xffffu);
   }
   const int rows = min(own, kMmRows);
@@ -213,6 +212,7 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
   uint16_t* const wp = mlds + S::WP;
   int32_t* const flag = reinterpret_cast<int32_t*>(mlds + S::FLAG);
   float* const slow_sum = reinterpret_cast<float*>(mlds + S::SUM);
+  float* const slow_taps = reinterpret_cast<float*>(mlds + S::TAPS);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -320,7 +320,8 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
   const int wc = tid >> 4, wk = tid & 15;  // this thread's channel and first tap of the weights
   float wv[NC + 1];
   mm_weights<NC>(p.w, p.w_dt, (int64_t)(c0 + wc) * W, wk, P, wv);
-  const float bias_v = p.has_bias ? kNegLog2e * ld_any(p.bias, c0 + (lane & 31), p.b_dt) : 0.0f;
+  const float bias_u = p.has_bias ? ld_any(p.bias, c0 + (lane & 31), p.b_dt) : 0.0f;
+  const float bias_v = kNegLog2e * bias_u;
 
   constexpr int XPAD = S::XP - (PP + kMmRows), GPAD = S::GP - (PP + kMmRows);
   for (int i = tid; i < kMmCh * XPAD; i += kMmNW * 64)
@@ -335,7 +336,8 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
   lds_barrier();
   uint32_t bad = 0;
   if (oct < 2 * NC) put(rw, xs, S::XP, 0, bad);
-  // Weights times -log2(e) (dsilu_scaled) in pieces, among the zeros.
+  // Weights times -log2(e) (dsilu_scaled) in pieces, among the zeros, and as they are for mm_slow.
+  if (tid < kMmCh) slow_taps[tid * S::SP + W] = bias_u;
   bool wbad = false;
 #pragma unroll
   for (int j = 0; j <= NC; ++j) {
@@ -343,6 +345,7 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
     if (k <= P) {
       uint16_t pc[3];
       wbad = !split3(kNegLog2e * wv[j], pc) || wbad;
+      slow_taps[wc * S::SP + k] = wv[j];
 #pragma unroll
       for (int i = 0; i < 3; ++i) wp[(wc * 3 + i) * S::WL + k + sh + 15] = pc[i];
     }
@@ -569,9 +572,7 @@ __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams
       const int n = __builtin_ctz(todo);
       const int ch = wave + n * kMmNW;
       tails_in(ch, lane);
-      mm_slow<NC>(xs + ch * S::XP, ys + ch * S::YP, g, wp + ch * 3 * S::WL, W,
-                  __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(bias_v), ch)), rows_t,
-                  own, lane,
+      mm_slow<NC>(xs + ch * S::XP, ys + ch * S::YP, g, slow_taps + ch * S::SP, W, rows_t, own, lane,
                   slow_sum + ch * S::SP,
                   [&](int r) { return with_dfinal ? dfinal(ch, r) : 0.0f; });
       // Whether the next step's window holds a g that is not finite.

@@ -1493,3 +1493,26 @@ def test_matrix_core_channels_do_not_see_each_other(W, B, T, D, c):
             assert torch.equal(got[k][..., others], clean[k][..., others]), (name, k)
         for k in ("dw", "db"):
             assert torch.equal(got[k][others], clean[k][others]), (name, k)
+
+
+@pytest.mark.parametrize("W", [33, 64, 120])
+def test_matrix_core_backward_of_large_finite_values(W):
+    """Weights and pre-activations above FLT_MAX / log2(e) = 2.36e38: the products' operands scaled by
+    log2(e) are infinite there, the values and their gradients are not."""
+    B, T, D = 2, 600, 64
+    inp = make_inputs(53 * W, B, T, D, W, init=True)
+    inp["w"][5, 2] = 2.5e38
+    for k in ("x", "init"):
+        inp[k][..., 5] *= 2.0 ** -124      # pre-activations of about 12
+    inp["dy"][..., 5] *= 0.1               # dx below 3.4e38
+    inp["w"][6, W - 1] = 1.0
+    inp["x"][0, 100, 6] = 3e38             # the pre-activation of its row
+    inp["dy"][0, 100:100 + W, 6] *= 0.1    # dweight below 3.4e38
+    gpu = run_gpu(inp, "silu", init_grad=True)
+    ref = oracle_ref(inp, True, need_dinit=True)
+    for k in ("out", "dx", "dinit"):
+        assert bool(gpu[k].isfinite().all()), k
+        check_lowp(gpu[k], ref[k], False, k)
+    for c in (np.arange(D) != 6, np.arange(D) == 6):  # channel 6 by itself: its dweight is about 1e37
+        check_sum(gpu["dw"][c], ref["dw"][c], "dweight")
+        check_sum(gpu["db"][c], ref["db"][c], "dbias")
