@@ -492,12 +492,6 @@ bool rows_ok(int x_dt, int cpl, int64_t T, int64_t D, const void* p, int64_t s_t
   return ((T - 1) * s_t + D) * esz < kMaxSlabBytes;
 }
 
-// Whether every row of an array starts on a multiple of the `cpl` channels a lane moves.
-bool rows_aligned(int x_dt, int cpl, int64_t D, const void* p, int64_t s_b, int64_t s_t) {
-  if (D % cpl || s_b % cpl || s_t % cpl) return false;
-  return reinterpret_cast<uintptr_t>(p) % (uintptr_t)(cpl * esize(x_dt)) == 0;
-}
-
 bool aligned_to(const void* p, int64_t bytes) {
   return (reinterpret_cast<uintptr_t>(p) % (uintptr_t)bytes) == 0;
 }
@@ -767,9 +761,9 @@ struct BwdPlan {
   size_t need = 0;     // workspace bytes the launches use
 };
 
-// Kernels, tiling and workspace of a backward with these rows (B, T, D > 0): the vectorised
-// kernels when the x dtype, the width and the alignment of every row of x, dout and dx (and of
-// dfinal_states) allow them, else the generic ones.
+// Kernels, tiling and workspace of a backward with these rows (B, T, D > 0): the matrix-core or the
+// vectorised kernels when the x dtype, the width, the channels and the extent of x, dout and dx allow
+// them (rows_ok; any row alignment does), else the generic ones.
 struct BwdPath {
   bool mfma = false;
   bool fast = false;
@@ -1015,16 +1009,6 @@ size_t ccv1d_bwd_workspace_bytes_for(const void* x, int64_t x_stride_b, int64_t 
         bwd_path(x, x_stride_b, x_stride_t, x_dtype, seq_idx != nullptr, dout, dout_stride_b,
                  dout_stride_t, dfinal_states, dx, T * D, D, true, mfma, B, T, D, W);
     if (path.need > need) need = path.need;
-  }
-  // Rows that do not start on the lanes' access width may be given to either family of kernels:
-  // the larger of their needs.
-  const int cpl = fast_dtype(x_dtype, W) ? bwd_shape(x_dtype, B, T, D, W).cpl : 1;
-  if (fast_dtype(x_dtype, W) &&
-      !(rows_aligned(x_dtype, cpl, D, x, x_stride_b, x_stride_t) &&
-        rows_aligned(x_dtype, cpl, D, dout, dout_stride_b, dout_stride_t) &&
-        rows_aligned(x_dtype, cpl, D, dx, T * D, D))) {
-    const size_t generic = partial_bytes(B * cdiv(T, kGenericL), W, D);
-    if (generic > need) return generic;
   }
   return need;
 }

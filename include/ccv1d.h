@@ -123,10 +123,11 @@ size_t ccv1d_bwd_workspace_bytes(int64_t batch, int64_t seqlen, int64_t dim, int
                                  int x_dtype);
 
 /* Bytes of device workspace ccv1d_bwd needs for these very tensors: the path its planner picks for
- * the alignment of x, dout, dfinal_states (may be NULL) and a contiguous dx (batch, seqlen, dim),
- * and a workspace aligned to 16 bytes (every torch allocation is). Never more than
- * ccv1d_bwd_workspace_bytes(batch, seqlen, dim, width, x_dtype), and often much less: that bound
- * covers the generic kernels' tiling (one partial row per 64 rows), which aligned rows never take.
+ * x, dout, dfinal_states (may be NULL) and a contiguous dx (batch, seqlen, dim), and a workspace
+ * aligned to 16 bytes (every torch allocation is). Where the activation or the type of the initial
+ * states decides between two paths (widths 33 to 128, bf16 x), the larger of their needs. Never more
+ * than ccv1d_bwd_workspace_bytes(batch, seqlen, dim, width, x_dtype), and often much less: that
+ * bound covers the shortest tiles of every path (one partial row per 64 rows).
  * Like the reference's partials allocation (causal_conv1d.py:493), sized from the launch it serves.
  * 0 for empty or invalid shapes. */
 size_t ccv1d_bwd_workspace_bytes_for(const void* x, int64_t x_stride_b, int64_t x_stride_t,

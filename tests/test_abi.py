@@ -75,19 +75,24 @@ def _ws_for(lib, x=1 << 20, sxb=None, sxt=None, xdt=2, seq=None, dy=1 << 24, dfi
 
 
 def test_workspace_bytes_for_the_call():
-    """The workspace of the path a call takes (its pointers' alignment and strides decide it): the
-    vectorised backward's partial rows for aligned rows, the generic kernels' bound otherwise; never
-    more than the shape-only upper bound. No pointer is dereferenced."""
+    """The workspace of the path a call takes: the vectorised backward's partial rows for rows of any
+    alignment and stride, the block kernels' for what those do not address; never more than the
+    shape-only upper bound. No pointer is dereferenced."""
     lib = _ffi.load()
     bound = lib.ccv1d_bwd_workspace_bytes(4, 8192, 1024, 4, 2)
     fast = _ws_for(lib)
     # the benchmark shape: 4 batch rows x 32 workgroups along time, (W + 1) x dim fp32 each
     assert fast == 4 * 32 * 5 * 1024 * 4
     assert fast < bound
-    # x misaligned by one element: the generic kernels, one partial row per 64-row tile
-    assert _ws_for(lib, x=(1 << 20) + 2) == 4 * (8192 // 64) * 5 * 1024 * 4 <= bound
-    # a time stride that is not a multiple of the channel vector: generic as well
-    assert _ws_for(lib, sxt=1027, sxb=8192 * 1027) == 4 * 128 * 5 * 1024 * 4
+    # x off by one element, a time stride that no access width divides, an odd dim: the same kernels
+    assert _ws_for(lib, x=(1 << 20) + 2) == fast
+    assert _ws_for(lib, sxt=1027, sxb=8192 * 1027) == fast
+    assert _ws_for(lib, D=1023) == 4 * 32 * 5 * 1023 * 4
+    # the block kernels, one partial row per segment: fp64 x, and a batch slab past 32-bit byte offsets
+    # (8 segments of 1024 rows); fewer channels than a lane takes (128 segments of 64 rows)
+    assert _ws_for(lib, xdt=3) == 4 * 8 * 5 * 1024 * 4
+    assert _ws_for(lib, xdt=0, sxt=(1 << 17) + 64, sxb=1 << 31) == 4 * 8 * 5 * 1024 * 4
+    assert _ws_for(lib, D=1) == 4 * 128 * 5 * 4
     # width above 128: partial rows plus the fp32 g buffer, as the shape-only bound says
     assert _ws_for(lib, B=2, T=300, D=100, W=129) == lib.ccv1d_bwd_workspace_bytes(2, 300, 100, 129, 2)
     # empty and invalid shapes
