@@ -15,8 +15,8 @@ Tolerances (from the build's north star):
     suite the largest deviation is 2.6e-6 rms(ref), and 1e-5 |ref| on entries above 0.1 rms(ref).
     In a bf16/fp16 parameter dtype the result is rounded, so rtol 1e-2 replaces 1e-3.
   * Bit-exact: padding positions give out == 0 and dx == 0, final_states == the last width-1 rows
-    of concat(initial_states, x), chunked forward == full forward, repeated backward gives the same
-    dweight/dbias bits.
+    of concat(initial_states, x), chunked forward == full forward (on the matrix cores at cuts of
+    whole 16 rows; elsewhere up to rounding), repeated backward gives the same dweight/dbias bits.
 BASELINE configurations 2-5 run at full size; the oracle (single-threaded C) checks a subset of
 channels there, which is exact because channels never interact in a depthwise convolution.
 """
@@ -1516,3 +1516,41 @@ def test_matrix_core_backward_of_large_finite_values(W):
     for c in (np.arange(D) != 6, np.arange(D) == 6):  # channel 6 by itself: its dweight is about 1e37
         check_sum(gpu["dw"][c], ref["dw"][c], "dweight")
         check_sum(gpu["db"][c], ref["db"][c], "dbias")
+
+
+@pytest.mark.parametrize("W", [33, 64, 128])
+def test_matrix_core_chunks_and_decode(W):
+    """A sequence in chunks with state handoff on the matrix cores. A row's sum is grouped by its place in
+    a block of 16 rows from the call's first one: chunks cut at multiples of 16 rows, in steps of 256
+    rows and of 512 (the uncut call), equal the uncut call bit for bit. At other cuts two
+    sums of 3 W products (W weights in three pieces) are off by at most 2^-23 of the sum of their
+    absolute values per addition, silu' is at most 1.1, and rounding to bf16 adds one ulp; results
+    that differ at all are rarer than 1 in 1000 (a difference of about sqrt(3 W) 2^-24 against the
+    spacing of bf16). The final states are exact always."""
+    B, T, D = 8, 1100, 2048
+    inp = make_inputs(59 * W, B, T, D, W, init=True)
+    x, w, b, init = (inp[k].to(DEV) for k in ("x", "w", "b", "init"))
+
+    def chunks(lengths):
+        state, outs, at = init, [], 0
+        for n in lengths:
+            o, state = causal_conv1d_fn(x[:, at:at + n], w, b, initial_states=state,
+                                        return_final_states=True, activation="silu")
+            outs.append(o)
+            at += n
+        return torch.cat(outs, dim=1), state, at
+
+    with torch.no_grad():
+        full, fin = causal_conv1d_fn(x, w, b, initial_states=init, return_final_states=True,
+                                     activation="silu")
+        got, state, _ = chunks((256, 16, 512, 48, 268))
+        assert torch.equal(got, full) and torch.equal(state, fin)
+        xx = torch.cat([init, x], dim=1)
+        got, state, n = chunks((7, 1, 1, 1, 1, 300, 1, 1))
+        assert torch.equal(state, xx[:, n:n + W - 1])
+        size = causal_conv1d_fn(x[:, :n].float().abs(), w.abs(), b.abs(),
+                                initial_states=init.float().abs())
+        a, f = got.float(), full[:, :n].float()
+        bound = 2.0 ** -7 * torch.maximum(a.abs(), f.abs()) + 1.1 * 3 * W * 2.0 ** -23 * size
+        assert bool(((a - f).abs() <= bound).all())
+        assert int((got != full[:, :n]).sum()) <= 1e-3 * got.numel()
