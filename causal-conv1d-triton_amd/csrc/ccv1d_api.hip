@@ -382,6 +382,15 @@ int64_t fill_rounds(int64_t T, int64_t cols, int64_t slots, int64_t unit, int64_
   return rows;
 }
 
+// The forward of a few rows at the narrowest widths (fp64 x, one channel) takes the scalar kernel, a row
+// per workgroup: a block kernel's start costs more than those rows (fp64, a decode step B=16 T=1
+// D=2048: W=2 6.8 -> 3.0 us, W=4 7.6 -> 4.1, W=8 6.3, where W=10 stays at about 8 on the block kernel;
+// T=16: W=4 8.2, W=8 9.6 on the block kernel). On grids past kScalarGroups workgroups, more rows each
+// (B=64 T=16 D=4096 W=2 25.3 -> 17.5).
+constexpr int64_t kScalarMaxW = 8;
+constexpr int64_t kScalarMaxTaps = 64;
+constexpr int64_t kScalarGroups = 16384;
+
 // Tiling of the kernels without compile-time widths. Above kMaxBlockW: tiles of kGenericL rows. Up
 // to it segments of the block kernels, whole steps: a CU holds as many workgroups as their LDS
 // allows, at most 4 in the forward and 2 in the backward (registers); the start (weights, window)
@@ -393,7 +402,11 @@ Tiling generic_tiling(int64_t B, int64_t T, int64_t D, int64_t W, int x_dt, bool
   static_assert(kGenericL % kBlkStep == 0, "segments are whole steps");
   Tiling t{};
   t.L = kGenericL;
-  if (W <= kMaxBlockW) {
+  if (!bwd && W <= kScalarMaxW && W * T <= kScalarMaxTaps) {
+    t.L = 1;
+    while (B * cdiv(D, 64) * cdiv(T, t.L) > kScalarGroups && t.L < T) t.L *= 2;
+    t.vec = 1;
+  } else if (W <= kMaxBlockW) {
     const int xs = esize(x_dt) == 2 ? 2 : 4;
     const int64_t fit = (160 << 10) / (int64_t)blk_lds_bytes((int)W, xs, bwd);
     const int64_t most = bwd ? 2 : 4;

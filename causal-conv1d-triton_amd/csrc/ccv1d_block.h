@@ -243,30 +243,32 @@ __global__ __launch_bounds__(kBlkNW * 64, 2) void fwd_block_kernel(const FwdPara
     put(own, r0, nxt);
     lds_barrier();
     if (a + kBlkStep < t1) rows.load(r0 + kBlkStep, nxt);
-    float z[kBlk];
-    // Rows of one sequence (the window's included): every mask is 1.
-    if (!sb || ring_one_id(sid, NB, slot, Pp - P, Pp + kBlk, lane)) {
-      block_conv(wl, xr, NB, slot, W, lane, z);
-    } else {
+    if (r0 < t1) {
+      float z[kBlk];
+      // Rows of one sequence (the window's included): every mask is 1.
+      if (!sb || ring_one_id(sid, NB, slot, Pp - P, Pp + kBlk, lane)) {
+        block_conv(wl, xr, NB, slot, W, lane, z);
+      } else {
+#pragma unroll
+        for (int r = 0; r < kBlk; ++r) {
+          const int32_t st = sid[ring_row(NB, slot, Pp + r)];
+          float v = wl[P * kBlkWPitch + lane] *
+                    static_cast<float>(xr[ring_row(NB, slot, Pp + r) * 64 + lane]);
+          for (int k = 0; k < P; ++k) {
+            const int q = ring_row(NB, slot, Pp + r - P + k);
+            if (sid[q] == st) v = fmaf(wl[k * kBlkWPitch + lane], static_cast<float>(xr[q * 64 + lane]), v);
+          }
+          z[r] = v;
+        }
+      }
 #pragma unroll
       for (int r = 0; r < kBlk; ++r) {
-        const int32_t st = sid[ring_row(NB, slot, Pp + r)];
-        float v = wl[P * kBlkWPitch + lane] *
-                  static_cast<float>(xr[ring_row(NB, slot, Pp + r) * 64 + lane]);
-        for (int k = 0; k < P; ++k) {
-          const int q = ring_row(NB, slot, Pp + r - P + k);
-          if (sid[q] == st) v = fmaf(wl[k * kBlkWPitch + lane], static_cast<float>(xr[q * 64 + lane]), v);
-        }
-        z[r] = v;
+        float v = z[r];
+        if (p.has_bias) v += bias;
+        if (sb && sid[ring_row(NB, slot, Pp + r)] < 0) v = 0.0f;
+        if (p.silu) v = v * sigmoid_f(v);
+        if (active && r0 + r < t1) ob[(int64_t)(r0 + r) * D] = to_store<TX>(v);
       }
-    }
-#pragma unroll
-    for (int r = 0; r < kBlk; ++r) {
-      float v = z[r];
-      if (p.has_bias) v += bias;
-      if (sb && sid[ring_row(NB, slot, Pp + r)] < 0) v = 0.0f;
-      if (p.silu) v = v * sigmoid_f(v);
-      if (active && r0 + r < t1) ob[(int64_t)(r0 + r) * D] = to_store<TX>(v);
     }
     lds_barrier();  // the step's oldest blocks are overwritten next
     slot += kBlkNW;
@@ -344,6 +346,11 @@ __global__ __launch_bounds__(kBlkNW * 64, 2) void bwd_block_kernel(const BwdPara
 #pragma unroll
     for (int q = 0; q < kBlk; ++q) dw[n][q] = 0.0f;
   float dwp = 0.0f, db = 0.0f;
+  // fp64 x comes here at every width: where the taps are one block, the waves share out the rows
+  // instead, and positions before the first tap are left out (fwd+bwd B=8 T=4096 D=1024 W=2 404 -> 374
+  // us, W=4 407 -> 378, W=16 436 -> 417).
+  const bool by_rows = sizeof(TX) == 8 && NC == 1;
+  static_assert(2 * kBlkNW * 64 + kBlkNW * kBlk * 64 <= blk_ring(2) * kBlk * 64, "sums in the g ring");
 
   int base = 0;  // slot of the block Pp rows before the step's first
   for (int a = t0; a - Pp < own_end; a += kBlkStep) {
@@ -451,13 +458,13 @@ __global__ __launch_bounds__(kBlkNW * 64, 2) void bwd_block_kernel(const BwdPara
       const bool one = !sb || ring_one_id(sid, NB, base, Pp - P, Pp + kBlkStep, lane);
 #pragma unroll
       for (int n = 0; n < NOWN; ++n) {
-        const int cb = wave + n * kBlkNW;
+        const int cb = by_rows ? n : wave + n * kBlkNW;
         if (cb >= NC) continue;
         float acc[kBlk];
 #pragma unroll
         for (int q = 0; q < kBlk; ++q) acc[q] = 0.0f;
 #pragma unroll 1
-        for (int i = 0; i < kBlkNW; ++i) {
+        for (int i = by_rows ? wave : 0; i < (by_rows ? wave + 1 : kBlkNW); ++i) {
           const int rows_left = own_end - (a + i * kBlk);
           if (rows_left <= 0) break;
           float gv[kBlk], lo[kBlk], hi[kBlk];
@@ -465,7 +472,16 @@ __global__ __launch_bounds__(kBlkNW * 64, 2) void bwd_block_kernel(const BwdPara
           if (one) {
             ring_block(xr, NB, base, i + cb, lane, lo);
             ring_block(xr, NB, base, i + cb + 1, lane, hi);
-            if (rows_left >= kBlk) {
+            if (by_rows && rows_left >= kBlk) {
+#pragma unroll
+              for (int q = 0; q < kBlk; ++q) {
+                if (q < Pp - P) continue;
+#pragma unroll
+                for (int r = 0; r < kBlk; ++r)
+                  acc[q] = fmaf(gv[r], q + r < kBlk ? lo[q + r < kBlk ? q + r : 0]
+                                                    : hi[q + r < kBlk ? 0 : q + r - kBlk], acc[q]);
+              }
+            } else if (rows_left >= kBlk) {
 #pragma unroll
               for (int r = 0; r < kBlk; ++r)
 #pragma unroll
@@ -507,17 +523,31 @@ __global__ __launch_bounds__(kBlkNW * 64, 2) void bwd_block_kernel(const BwdPara
   // the g ring after them, is free now).
   wl[wave * 64 + lane] = dwp;
   wl[(kBlkNW + wave) * 64 + lane] = db;
+  float* const waves = gr + 2 * kBlkNW * 64;  // [wave][position][64], by_rows
+  if (by_rows) {
+#pragma unroll
+    for (int q = 0; q < kBlk; ++q) waves[(wave * kBlk + q) * 64 + lane] = dw[0][q];
+  }
   lds_barrier();
   float* pp = p.part + ((int64_t)b * p.tl.nT + tile) * (W + 1) * D + c;
   if (!active) return;
   const int sh = Pp - P;
+  if (by_rows) {
+    for (int q = sh + wave; q < kBlk; q += kBlkNW) {
+      float s = waves[q * 64 + lane];
 #pragma unroll
-  for (int n = 0; n < NOWN; ++n)
-#pragma unroll
-    for (int q = 0; q < kBlk; ++q) {
-      const int k = (wave + n * kBlkNW) * kBlk + q - sh;
-      if (k >= 0 && k < P) pp[(int64_t)k * D] = dw[n][q];
+      for (int v = 1; v < kBlkNW; ++v) s += waves[(v * kBlk + q) * 64 + lane];
+      pp[(int64_t)(q - sh) * D] = s;
     }
+  } else {
+#pragma unroll
+    for (int n = 0; n < NOWN; ++n)
+#pragma unroll
+      for (int q = 0; q < kBlk; ++q) {
+        const int k = (wave + n * kBlkNW) * kBlk + q - sh;
+        if (k >= 0 && k < P) pp[(int64_t)k * D] = dw[n][q];
+      }
+  }
   if (wave == 0 || (wave == 1 && p.has_bias)) {
     float s = wl[wave * kBlkNW * 64 + lane];
 #pragma unroll

@@ -21,7 +21,8 @@ struct Tiling {
   int32_t nGW;   // wave columns: ceil(D / VEC / 64)
   int32_t nTB;   // workgroups along time per batch row: ceil(nT / NW)
   int32_t nBlk;  // workgroups in the grid: B * nGW * nTB
-  int32_t vec;   // channels per lane the tiling was made for (0 for the generic kernels)
+  int32_t vec;   // channels per lane the tiling was made for (0 for the generic kernels,
+                 // 1 for the scalar forward at the block kernels' widths)
   // Workgroup order: 0 = time fastest (a wave column's consecutive time tiles are consecutive
   // workgroups), 1 = wave column fastest (the columns of one range of rows are), for rows that are
   // not aligned to the 128-byte line, whose lines straddle neighbouring columns (TileCoord).

@@ -39,7 +39,7 @@ static hipError_t bwd_block(const BwdParams& p, hipStream_t s) {
 
 template <typename TX>
 hipError_t launch_fwd_generic_t(const FwdParams& p, hipStream_t s) {
-  if (p.W <= kMaxBlockW) {
+  if (p.W <= kMaxBlockW && p.tl.vec == 0) {  // vec == 1: few rows, the scalar kernel
     if constexpr (sizeof(TX) == 2) {
       if (ring_of_tx<TX>(p)) return fwd_block<TX, TX>(p, s);
     }

@@ -1554,3 +1554,36 @@ def test_matrix_core_chunks_and_decode(W):
         bound = 2.0 ** -7 * torch.maximum(a.abs(), f.abs()) + 1.1 * 3 * W * 2.0 ** -23 * size
         assert bool(((a - f).abs() <= bound).all())
         assert int((got != full[:, :n]).sum()) <= 1e-3 * got.numel()
+
+
+@pytest.mark.parametrize("W", [2, 4, 5, 8, 9])
+@pytest.mark.parametrize("xdt,D", [(torch.float64, 70), (torch.bfloat16, 1)])
+def test_few_rows_outside_the_vectorised_kernels(W, xdt, D):
+    """fp64 x and single channels: calls of up to 64 / W rows take the scalar forward (to width 8), longer
+    ones the block kernel. Row counts around that limit give the first rows of a long call bit for bit,
+    final states included; so does a grid on which the scalar kernel takes several rows each."""
+    for B, D, lengths in ((2, D, sorted({1, 2, 64 // W, 64 // W + 1})), (65, 4100, (64 // W,))):
+        if D > 1000 and xdt != torch.float64:
+            continue
+        inp = make_inputs(61 * W + D, B, 70, D, W, xdt=xdt, init=True)
+        x, w, b, init = (inp[k].to(DEV) for k in ("x", "w", "b", "init"))
+        xx = torch.cat([init, x], dim=1)
+        for act in (None, "silu"):
+            full = causal_conv1d_fn(x, w, b, initial_states=init, activation=act)
+            for T in lengths:
+                out, fin = causal_conv1d_fn(x[:, :T], w, b, initial_states=init,
+                                            return_final_states=True, activation=act)
+                assert torch.equal(out, full[:, :T]) and torch.equal(fin, xx[:, T:T + W - 1])
+
+
+@pytest.mark.parametrize("W", [2, 9, 16, 17, 18])
+def test_fp64_backward_of_one_tap_block(W):
+    """fp64 x to width 17: the backward's waves share out the rows and add their dweight sums up."""
+    for T in (5, 64, 200):
+        inp = make_inputs(67 * W + T, 2, T, 70, W, xdt=torch.float64, init=True)
+        gpu = run_gpu(inp, "silu", return_final=True, dfinal=True, init_grad=True)
+        compare(gpu, oracle_ref(inp, True, final=True, dfinal=True, need_dinit=True), True)
+    ids = varlen_seq(W, 2, 500, lo=20, hi=90)
+    inp = make_inputs(71 * W, 2, 500, 70, W, xdt=torch.float64, init=True, seq=ids)
+    gpu = run_gpu(inp, None, init_grad=True)
+    compare(gpu, oracle_ref(inp, False, need_dinit=True), False)
