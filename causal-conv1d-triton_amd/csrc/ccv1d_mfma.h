@@ -97,6 +97,7 @@ static_assert(kMmNW == 8 && kMmCh == 32, "every fourth bit of a half");
 // The wave's channels whose staged rows hold an infinity or NaN: a thread has rows of channels
 // 2 (lane % 16) and the one after it, `bad` says so of them in bits 15 and 31.
 __device__ __forceinline__ uint32_t mm_bad_rows(uint32_t bad) {
+  if (!__any((bad & 0x80008000u) != 0)) return 0;
   const uint64_t e = __ballot((bad & 0x8000u) != 0), o = __ballot((bad & 0x80000000u) != 0);
   uint32_t lo = (uint32_t)e | (uint32_t)(e >> 32), hi = (uint32_t)o | (uint32_t)(o >> 32);
   lo |= lo >> 16;
@@ -107,6 +108,7 @@ __device__ __forceinline__ uint32_t mm_bad_rows(uint32_t bad) {
 // Those whose weights do: 16 lanes have the taps of one of the wave's 4 channels.
 __device__ __forceinline__ uint32_t mm_bad_taps(bool bad, int wave) {
   const uint64_t b = __ballot(bad);
+  if (b == 0) return 0;
   uint32_t set = 0;
 #pragma unroll
   for (int q = 0; q < 4; ++q)

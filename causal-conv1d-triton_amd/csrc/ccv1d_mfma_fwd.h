@@ -18,6 +18,8 @@
 // kernel takes 14.2 us, at 24 11.0.
 #pragma once
 
+#include <type_traits>
+
 #include "ccv1d_mfma.h"
 
 namespace ccv1d {
@@ -187,13 +189,12 @@ __global__ __launch_bounds__(kMmNW * 64, 4) void fwd_mfma_kernel(const FwdParams
     const uint32_t slow = mm_wave_bits((uint32_t)(slow_prev | f), wave);
     slow_prev = f;
 
-#pragma unroll
-    for (int n = 0; n < kMmPerWave; ++n) {
+    auto channel = [&](int n, auto by_row) {
       const int ch = wave + n * kMmNW;
       uint16_t* const xc = xs + ch * S::XP;
       const float bias = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(bias_v), ch));
       float o[SUB][4];
-      if (!(slow >> (4 * n) & 1)) {
+      if constexpr (!decltype(by_row)::value) {
         // 8 weights of a lane from any element on: aligned words, shifted where the start is odd.
         const uint32_t* const wq = reinterpret_cast<const uint32_t*>(
             wp + ch * 3 * S::WL + ((8 * lq - li + 15) & ~1));
@@ -254,6 +255,17 @@ __global__ __launch_bounds__(kMmNW * 64, 4) void fwd_mfma_kernel(const FwdParams
         *reinterpret_cast<u32x2*>(xc + PP + h * kMmRows + 16 * li + 4 * lq) =
             u32x2{bf_pack(o[h][0], o[h][1]), bf_pack(o[h][2], o[h][3])};
       mm_fence();
+    };
+    // Without a branch between the channels where no channel needs it.
+    if ((slow & 0x1111u) == 0) {
+#pragma unroll
+      for (int n = 0; n < kMmPerWave; ++n) channel(n, std::false_type{});
+    } else {
+#pragma unroll 1
+      for (int n = 0; n < kMmPerWave; ++n) {
+        if (slow >> (4 * n) & 1) channel(n, std::true_type{});
+        else channel(n, std::false_type{});
+      }
     }
     lds_barrier();
 
