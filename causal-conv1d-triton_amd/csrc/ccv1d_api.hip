@@ -429,6 +429,29 @@ bool mfma_takes(int x_dt, int64_t D, int64_t W, bool silu, bool seq, bool init, 
          (!init || i_dt == x_dt);
 }
 
+// Whether they are the faster ones for these sizes. A step is 256 rows of 32 channels however few rows
+// a call has, so short rows of many channels take many rounds of almost empty steps; the block
+// kernels' are 64 rows of 64 channels. Both sides measured (bf16, silu; block against matrix cores):
+//   backward, more than one round of channel blocks, fwd+bwd: to 192 rows where a CU holds two of the
+//   block kernel's workgroups (to width 81), B=64 D=4096 W=64 T=1 213 against 826 us, T=192 591
+//   against 848 (T=256 732 against 1084, but the matrix cores' dweight is 1-6 % closer to its 64-bit
+//   value there; B=16 T=512 D=1024 W=33 98 against 79); to 64 rows where it holds one, B=8 T=64
+//   D=4096 W=128 118 against 191 (B=4 T=128 D=5376 183 against 156). In one round the matrix cores win
+//   or tie (B=4 T=1 D=2048 W=64 35 against 37, B=1 T=64 D=1024 38.5 against 34).
+//   forward, calls under 16 rows (decode steps): past two rounds where a CU holds four of the block
+//   kernel's workgroups, B=64 T=1 D=4096 W=33 30 against 72, W=64 38 against 93, with states B=32
+//   W=64 43 against 52 (B=16 D=2048 W=48 15.4 against 14.0; W=96 with states B=32 D=4096 88 against
+//   63). Longer ones stay on the matrix cores (B=64 D=4096 W=64 T=64 55 against 91, T=128 even), so
+//   that chunks cut at multiples of 16 rows keep the uncut call's bits.
+constexpr int64_t kMmBwdShort = 192, kMmBwdShortAlone = 64, kMmFwdShort = 16;
+bool mfma_pays(int64_t B, int64_t T, int64_t D, int64_t W, bool bwd) {
+  const int64_t cols = B * cdiv(D, kMmCh);
+  const int64_t fit = (160 << 10) / (int64_t)blk_lds_bytes((int)W, 2, bwd);
+  if (cdiv(D, 64) > 65535) return true;  // past the block kernels' grid
+  if (bwd) return cols <= 256 || T > (fit >= 2 ? kMmBwdShort : kMmBwdShortAlone);
+  return T >= kMmFwdShort || cols <= 1024 || fit < 4;
+}
+
 // Its tiling: one workgroup per CU at a time; a segment and its window are walked in whole steps, and
 // the start and end (weights, sums) cost about one more. (With the longest segments of 8 steps that
 // still filled the chip, rows left over ran a second round: B=2 T=4096 D=1024 W=64 170 -> 115 us.) Only
@@ -599,6 +622,7 @@ int fwd_entry(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype
   const bool mfma = T > 0 &&
                     mfma_takes(x_dtype, D, W, silu != 0, seq_idx != nullptr,
                                initial_states != nullptr, init_dtype) &&
+                    mfma_pays(B, T, D, W, false) &&
                     rows_ok(x_dtype, 2, T, D, x, x_stride_t) && rows_ok(x_dtype, 2, T, D, out, D) &&
                     (!final_states || aligned_to(final_states, esize(x_dtype))) &&
                     B * cdiv(D, kMmCh) * cdiv(T, kGenericL) < (int64_t(1) << 31);
@@ -793,7 +817,7 @@ BwdPath bwd_path(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dt
                  int64_t dx_stride_t, bool ws_aligned, bool mfma, int64_t B, int64_t T, int64_t D,
                  int64_t W) {
   BwdPath r;
-  r.mfma = mfma && rows_ok(x_dtype, 2, T, D, x, x_stride_t) &&
+  r.mfma = mfma && mfma_pays(B, T, D, W, true) && rows_ok(x_dtype, 2, T, D, x, x_stride_t) &&
            rows_ok(x_dtype, 2, T, D, dout, dout_stride_t) &&
            rows_ok(x_dtype, 2, T, D, dx, dx_stride_t) &&
            (!dfinal_states || aligned_to(dfinal_states, esize(x_dtype))) && ws_aligned;

@@ -8,7 +8,7 @@
 // channel with infinities or NaN in reach is computed row by row, by its own values alone as in the
 // backward. A row's sum is grouped by its place in its block of 16 rows from the call's first row on
 // (segments are multiples of 16), whatever the segment: chunks cut elsewhere round about 1 value of
-// out in 10^4 differently.
+// out in 10^4 differently (so do calls under 16 rows, which mfma_pays may give to the block kernels).
 //
 // Measured, forward alone B=2 T=4096 D=1024 against fwd_block_kernel: W=33 21.8 -> 13.2 us, W=64
 // 30.3 -> 14.8, W=128 47 -> 18.4 (memory: about 6). What bounds it is LDS reads and vector work around

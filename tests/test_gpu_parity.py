@@ -1587,3 +1587,15 @@ def test_fp64_backward_of_one_tap_block(W):
     inp = make_inputs(71 * W, 2, 500, 70, W, xdt=torch.float64, init=True, seq=ids)
     gpu = run_gpu(inp, None, init_grad=True)
     compare(gpu, oracle_ref(inp, False, need_dinit=True), False)
+
+
+@pytest.mark.parametrize("W,B,T,D", [(33, 33, 15, 1024), (33, 33, 16, 1024), (64, 17, 1, 2048),
+                                     (64, 9, 192, 1024), (64, 9, 193, 1024), (81, 9, 192, 1001),
+                                     (82, 9, 65, 1001), (113, 9, 64, 1024), (113, 8, 64, 1024)])
+def test_matrix_core_or_block_kernels_for_short_rows(W, B, T, D):
+    """bf16 with silu on both sides of the rule for short rows of many channels: forwards under 16 rows past
+    1024 channel blocks, backwards of up to 192 rows (64 from width 82) past 256."""
+    inp = make_inputs(73 * W + T, B, T, D, W, init=True)
+    gpu = run_gpu(inp, "silu", return_final=True, dfinal=True, init_grad=True)
+    cols = _cols(D, 6, W)
+    compare(gpu, oracle_ref(inp, True, cols=cols, final=True, dfinal=True, need_dinit=True), True, cols)
