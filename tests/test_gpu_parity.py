@@ -1599,3 +1599,28 @@ def test_matrix_core_or_block_kernels_for_short_rows(W, B, T, D):
     gpu = run_gpu(inp, "silu", return_final=True, dfinal=True, init_grad=True)
     cols = _cols(D, 6, W)
     compare(gpu, oracle_ref(inp, True, cols=cols, final=True, dfinal=True, need_dinit=True), True, cols)
+
+
+@pytest.mark.parametrize("B,T,D,W", [(16, 100, 512, 33), (8, 64, 1024, 64), (2, 4096, 1024, 64)])
+def test_matrix_core_dweight_is_no_further_off_than_the_vector_sums(B, T, D, W):
+    """dweight of the matrix cores against its 64-bit value is no further off than that of the block
+    kernels, which the same call takes with (zero) initial states of another type. The first two shapes
+    have one step per row of the batch, the third several."""
+    inp = make_inputs(79 * W + T, B, T, D, W)
+    x, w, b, dy = (inp[k].to(DEV) for k in ("x", "w", "b", "dy"))
+    xd, wd, yd = x.double(), w.double(), dy.double()
+    xp = torch.cat([xd.new_zeros(B, W - 1, D), xd], dim=1)
+    z = b.double().expand(B, T, D).clone()
+    for k in range(W):
+        z += wd[:, k] * xp[:, k:k + T]
+    s = torch.sigmoid(z)
+    g = yd * s * (1 + z * (1 - s))
+    want = torch.stack([(g * xp[:, k:k + T]).sum((0, 1)) for k in range(W)], dim=1)
+
+    def error(init):
+        wr = w.clone().requires_grad_(True)
+        out = causal_conv1d_fn(x, wr, b, initial_states=init, activation="silu")
+        (dw,) = torch.autograd.grad(out, wr, dy)
+        return float((dw.double() - want).norm() / want.norm())
+
+    assert error(None) <= error(torch.zeros(B, W - 1, D, device=DEV))
