@@ -14,7 +14,9 @@ check:
   fits 4 waves per SIMD (at most 128 VGPRs of the 512 a SIMD gives each lane); from width 21 the
   one-channel backward holds 3 or 2 by design (its dweight sums and windows of W taps);
 * with fp32 x and no seq_idx, the forward at every width and the backward up to width 4 fit
-  4 waves per SIMD.
+  4 waves per SIMD;
+* the matrix-core and block forwards fit 4 waves per SIMD, their backwards 2, as their tilings
+  assume, with one instance for each count of 16-row window blocks.
 
 The objects are built by `make -C causal-conv1d-triton_amd` (or `__graft_entry__.build()`); the
 tests skip when they or the LLVM tools of the ROCm install are absent.
@@ -148,6 +150,20 @@ def test_fp32_kernels_hold_four_waves_per_simd(kernels):
         if _waves_per_simd(v) < 4:
             bad.append((d["name"], v))
     assert not bad, f"below 4 waves per SIMD: {bad}"
+
+
+def test_matrix_core_and_block_kernels_hold_their_waves(kernels):
+    found, bad = {}, []
+    for _, d in kernels:
+        m = re.match(r"_ZN5ccv1d1[56](fwd|bwd)_(mfma|block)_kernelI(\w+?)EEv", d["name"])
+        if not m:
+            continue
+        found.setdefault(m.group(1, 2), []).append(m.group(3))
+        if _waves_per_simd(int(d["vgpr_count"])) < (4 if m.group(1) == "fwd" else 2):
+            bad.append((d["name"], d["vgpr_count"]))
+    assert not bad, f"fewer waves than the tilings assume: {bad}"
+    assert len(found["bwd", "mfma"]) == 7 and len(found["fwd", "mfma"]) == 14
+    assert len(found["fwd", "block"]) == len(found["bwd", "block"]) == 6
 
 
 def test_waves_per_simd_formula():
