@@ -420,9 +420,9 @@ Tiling generic_tiling(int64_t B, int64_t T, int64_t D, int64_t W, int x_dt, bool
   return t;
 }
 
-// The matrix-core kernels (ccv1d_mfma.h, ccv1d_mfma_fwd.h): bf16 x with silu, without seq_idx, and initial states (if
-// any) of x's dtype. Without an activation the vector kernels stay: their results are the reference's
-// operation order bit for bit.
+// The matrix-core kernels (ccv1d_mfma.h, ccv1d_mfma_fwd.h): bf16 x with silu, without seq_idx, and
+// initial states (if any) of x's dtype. Without an activation the vector kernels stay: their
+// results are the reference's operation order bit for bit.
 constexpr int64_t kMmMinW = kMaxFastW + 1;  // see ccv1d_mfma.h
 bool mfma_takes(int x_dt, int64_t D, int64_t W, bool silu, bool seq, bool init, int i_dt) {
   return x_dt == CCV1D_BF16 && silu && !seq && W >= kMmMinW && W <= kMaxBlockW && D >= kMmCh &&
@@ -467,10 +467,11 @@ Tiling mfma_tiling(int64_t B, int64_t T, int64_t D, int64_t W) {
   return t;
 }
 
-// The forward's: two workgroups per CU (with as many as the LDS holds, 3 or 4, the shorter segments
-// they get cost more than the rounds saved: B=2 T=4096 D=1024 W=64 16.6 -> 21.1 us); segments above
-// 256 rows take steps of 512, which share the weights' fragments (16.6 -> 15.0 us) and cost 1.75
-// steps of 256; the start costs about one.
+// The forward's: two workgroups per CU, which is what the LDS holds of the kernel in steps of 512 rows
+// from 4 window blocks on (3 below). Of the kernel in steps of 256 rows it holds 4 to 2, but the shorter
+// segments of such a tiling cost more than the rounds saved (B=2 T=4096 D=1024 W=64, steps of 256
+// rows and 3 workgroups 16.6 -> 21.1 us). Segments above 256 rows take steps of 512, which share the
+// weights' fragments (16.6 -> 14.8 us) and cost 1.75 steps of 256; the start costs about one.
 Tiling mfma_fwd_tiling(int64_t B, int64_t T, int64_t D, int64_t W) {
   Tiling t{};
   const int64_t window = blk_window((int)W);

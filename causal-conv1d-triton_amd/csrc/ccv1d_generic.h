@@ -1,7 +1,8 @@
 // Scalar kernels for widths above kMaxBlockW (128; ccv1d_block.h has the narrower ones that no
-// vectorised instance covers). One lane owns one channel of one tile; the lanes of a wave cover 64
-// consecutive channels, so every row access is coalesced. Also: the deterministic partial-sum
-// reduction and the small fill/copy kernel used by the empty-sequence paths.
+// vectorised instance covers, except the forward of a few rows: generic_tiling). One lane owns one
+// channel of one tile; the lanes of a wave cover 64 consecutive channels, so every row access is
+// coalesced. Also: the deterministic partial-sum reduction and the small fill/copy kernel used by
+// the empty-sequence paths.
 #pragma once
 
 #include "ccv1d_device.h"

@@ -85,7 +85,7 @@ constexpr int kFwdLongW = 17;
 constexpr int kBwdLongW = 11;
 constexpr int kCplLong = 1;
 constexpr int kReduceNW = 16;    // waves per reduction workgroup
-constexpr int kGenericL = 64;    // rows per tile of the kernels above kMaxBlockW
+constexpr int kGenericL = 64;    // rows per tile above kMaxBlockW, of the shortest segments below it
 
 // Timing events of the calling thread (ccv1d_time_main_kernel). `pending` holds a request for the
 // thread's next entry-point call, which takes it; the call sets `armed` right before its main kernel

@@ -29,9 +29,11 @@
 // rounds and the matrix-core forward at 68.5, 85.7, 107.6 and 121.7, the weights' fragments kept from z
 // to dx (64.9, 82.2, 101.7) and no dweight products in a segment's last step where that holds dx rows
 // alone (63.7, 80.5, 98.7, 119.1; leaving z out there too past the end of x: T=256 W=40 121.4 -> 118.2, but
-// W=33 63.7 -> 64.4). What bounds it is the vector
-// work around the products (silu', the pieces, addresses: about 200 instructions per 256 elements)
-// at one workgroup per CU (the dweight tiles' registers); at widths 9-32 the register-window kernels
+// W=33 63.7 -> 64.4). These are graphs of many steps; one step per graph replay takes 85 us at W=64.
+// What bounds it is latency: at W=64 (66 us under the counters) the matrix units are busy 9 us, the
+// vector units about 17 (504 instructions per 256 elements), LDS 26 (8 of them bank conflicts), and the
+// waves wait 45 % of their time, 2 per SIMD in phases between barriers. A second workgroup per CU
+// fits neither the LDS (from NC = 3) nor the registers. At widths 9-32 the register-window kernels
 // are faster (B=4 T=8192 D=1024 W=16 95 us against 150, W=32 159 against 210).
 #pragma once
 
@@ -202,7 +204,8 @@ __device__ __forceinline__ void mm_slow(const uint16_t* xc, uint16_t* yc, uint16
   mm_fence();
 }
 
-// Two waves per SIMD: the dweight tiles alone take 16 (NC + 1) registers.
+// Two waves per SIMD: the dweight tiles alone take 16 (NC + 1) registers, and LDS from NC = 3 on holds
+// one workgroup per CU.
 template <int NC>
 __global__ __launch_bounds__(kMmNW * 64, 2) void bwd_mfma_kernel(const BwdParams p) {
   using S = MmShape<NC>;

@@ -11,8 +11,9 @@
 // out in 10^4 differently (so do calls under 16 rows, which mfma_pays may give to the block kernels).
 //
 // Measured, forward alone B=2 T=4096 D=1024 against fwd_block_kernel: W=33 21.8 -> 13.2 us, W=64
-// 30.3 -> 14.8, W=128 47 -> 18.4 (memory: about 6). What bounds it is LDS reads and vector work around
-// the products: the weights' fragments start at any element, 5 words and 4 shifts each, so segments
+// 30.3 -> 14.8, W=128 47 -> 18.4 (memory: about 6). No unit is busy half of that at W=64 (LDS 5 us,
+// vector instructions 3.3, matrix units 2; the waves wait 38 % of their time on memory and LDS and
+// 35 % to issue). The weights' fragments start at any element, 5 words and 4 shifts each, so segments
 // above 256 rows take steps of SUB = 2 and use each fragment twice (W=64 16.6 -> 14.8 us); below, half
 // of such a step would be empty (B=1 T=512 W=64 6.6 us against 8.6). At width 32 the register-window
 // kernel takes 14.2 us, at 24 11.0.

@@ -49,8 +49,7 @@ def test_workspace_bytes():
     assert lib.ccv1d_bwd_workspace_bytes(1, 0, 8, 4, 2) == 0
     assert lib.ccv1d_bwd_workspace_bytes(1, 10, 8, 1, 2) == 0
     n = lib.ccv1d_bwd_workspace_bytes(4, 8192, 1024, 4, 2)
-    # never less than the generic kernel's one fp32 partial row of (width + 1) * dim floats per
-    # 64-row tile
+    # never less than one fp32 partial row of (width + 1) * dim floats per 64 rows
     assert n >= 4 * (8192 // 64) * 5 * 1024 * 4
     # whole fp32 partial rows of (width + 1) * dim floats
     assert n % (5 * 1024 * 4) == 0

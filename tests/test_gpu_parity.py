@@ -216,9 +216,8 @@ def test_channel_counts(D):
 @pytest.mark.parametrize("D", [1002, 260])
 @pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float32])
 def test_wide_widths_channel_counts(W, D, xdt):
-    """Widths from 6 keep 2 channels per lane in the backward: D = 1002 (not a multiple of 4, so
-    the forward takes the generic kernel while the backward stays vectorised) and D = 260 (a last
-    wave column that is mostly empty)."""
+    """Widths from 6 keep 2 channels per lane in the backward: D = 1002 (not a multiple of the 4 channels
+    that the forward may take) and D = 260 (a last wave column that is mostly empty)."""
     inp = make_inputs(W * 10 + D, 3, 333, D, W, xdt=xdt, init=True)
     gpu = run_gpu(inp, "silu", return_final=True, dfinal=True, init_grad=True)
     compare(gpu, oracle_ref(inp, True, final=True, dfinal=True, need_dinit=True), True)
@@ -230,8 +229,8 @@ def test_dtypes(xdt, wdt):
     """Every x dtype against every weight/bias dtype, with initial states in a third dtype (fp32
     for fp32 weights, the other 16-bit type for 16-bit weights), so the conversions on load and
     the stores of dweight, dbias and the initial-state gradient in their own dtype all run; widths
-    4 (vectorised kernels and, with a dim that is not a multiple of 4, the generic ones), 12 and 20
-    (one channel per lane). Without the activation out, dx and dinit must be bit-identical to the
+    4 (also with a dim that is not a multiple of 4), 12 and 20 (one channel per lane); fp64 x on the block
+    kernels. Without the activation out, dx and dinit must be bit-identical to the
     oracle's fp32 values rounded once to their dtype."""
     idt = {torch.float32: torch.float32, torch.bfloat16: torch.float16,
            torch.float16: torch.bfloat16}[wdt]
@@ -523,7 +522,7 @@ def test_native_backward_refuses_foreign_gradients():
 
 
 @pytest.mark.parametrize("case", ["plain", "states", "seq_int64", "strided", "final_out",
-                                  "generic", "empty"])
+                                  "wide", "empty"])
 def test_native_inference_forward_matches_python_path(case):
     """Inference calls (no autograd) go through one native call (_ccv1d_torch: checks,
     canonicalisation, allocation, launch). The same call made from Python (the ctypes binding
@@ -533,7 +532,7 @@ def test_native_inference_forward_matches_python_path(case):
 
     assert _ffi._torch_native is not None
     B, T, D, W = 3, 257, 256, 4
-    if case == "generic":
+    if case == "wide":
         W = 20
     if case == "empty":
         T = 0
@@ -572,7 +571,7 @@ def test_native_inference_forward_matches_python_path(case):
 
 @pytest.mark.parametrize("W,xdt", [(4, torch.bfloat16), (12, torch.bfloat16), (4, torch.float64)])
 def test_kernel_timing_events(W, xdt):
-    """ccv1d_time_main_kernel (fast and generic kernels): the timed launch gives bit-identical
+    """ccv1d_time_main_kernel (vectorised and block kernels): the timed launch gives bit-identical
     results, sets both events to a positive kernel time inside the interval of events recorded
     around the call, and covers one call only (an untimed call after it leaves the events as they
     were)."""
@@ -760,9 +759,9 @@ def test_forward_cache_policies_leave_results_unchanged(case):
                                    (64, torch.float32), (100, torch.bfloat16), (100, torch.float32),
                                    (128, torch.bfloat16), (128, torch.float32), (20, torch.float64)])
 def test_generic_ring_widths(W, xdt):
-    """Widths 33-128 (and fp64 x from width 2) run the generic kernels with their weights and row
-    windows in LDS; from width 64 the backward's LDS exceeds the default 64 KiB and the launcher
-    raises the kernel's limit. Against the oracle around the window length, with initial and final
+    """Widths 33-128 run the block kernels or, bf16 x with silu and no seq_idx, the matrix-core ones, fp64
+    x from width 2 the block kernels; where a kernel's LDS exceeds the default 64 KiB the launcher raises
+    its limit. Against the oracle around the window length, with initial and final
     states and their gradients, and with seq_idx."""
     D = 72
     for T in (1, W - 1, W + 1, 300):
@@ -1212,8 +1211,8 @@ def test_concurrent_streams():
 def test_graph_replays_match_eager(B, T, D, W):
     """fwd+bwd captured in a HIP graph and replayed several times, with the program's own eager work
     and synchronisations in between; every replay must equal the eager result bit for bit. Widths
-    64 and 128 run the generic ring kernels, whose LDS above 64 KiB is allowed once per device on
-    their first launch, so the captured launches make no runtime call for it."""
+    64 and 128 run the matrix-core kernels, whose LDS above 64 KiB is allowed once per device on their
+    first launch, so the captured launches make no runtime call for it."""
     inp = make_inputs(33, B, T, D, W, init=True)
     x = inp["x"].to(DEV).requires_grad_(True)
     w = inp["w"].to(DEV).requires_grad_(True)
@@ -1250,24 +1249,23 @@ def test_graph_replays_match_eager(B, T, D, W):
 # projection output's gradient).
 # ------------------------------------------------------------------------------------------------
 
-@pytest.mark.parametrize("case", ["aligned", "odd_offset", "generic_width", "wide_width", "seq_idx",
+@pytest.mark.parametrize("case", ["aligned", "odd_offset", "long_width", "wide_width", "seq_idx",
                                   "states", "straddling"])
 def test_backward_into_strided_dx(case):
     """causal_conv1d_bwd writes dx into channels [c0, c0 + dim) of a wider buffer: the same bits
-    as the contiguous backward, and every other element of the buffer untouched. At an odd channel
-    offset dx's rows are not aligned for the vectorised kernels, so the generic kernels run; their
-    rounding differs from the vectorised ones', and that case is held to the tolerances."""
+    as the contiguous backward, and every other element of the buffer untouched, at an odd channel
+    offset too."""
     from causal_conv1d_triton.causal_conv1d import _bwd
     from causal_conv1d_triton.fused import causal_conv1d_bwd
 
     B, T, D, W, c0, wide = 2, 700, 512, 4, 512, 1536
     if case == "odd_offset":
-        c0 = 3                       # rows misaligned for the vectorised kernels: generic path
+        c0 = 3
     if case == "straddling":
         # a 3104-byte pitch: rows start 0, 32, 64 or 96 bytes into a 128-byte line, so the
         # backward takes the column-fastest workgroup order and non-temporal dx stores
         wide = 1552
-    if case == "generic_width":
+    if case == "long_width":
         W = 20
     if case == "wide_width":
         W, T, D = 200, 300, 64
@@ -1286,15 +1284,8 @@ def test_backward_into_strided_dx(case):
     want = _bwd(x, w, b, sq, s0, dy, dfin, init, True)
     torch.cuda.synchronize()
     assert dx.data_ptr() == view.data_ptr()
-    if case == "odd_offset":
-        torch.testing.assert_close(view.float(), want[0].float(), rtol=1e-2, atol=1e-2)
-        # The generic kernels sum dweight/dbias over other tiles: fp32 rounding apart.
-        for got, ref in ((dw, want[1]), (db, want[2])):
-            rms = ref.double().pow(2).mean().sqrt().item()
-            torch.testing.assert_close(got, ref, rtol=1e-3, atol=1e-5 * rms + 1e-7)
-    else:
-        assert torch.equal(view, want[0]), case
-        assert torch.equal(dw, want[1]) and torch.equal(db, want[2]), case
+    assert torch.equal(view, want[0]), case
+    assert torch.equal(dw, want[1]) and torch.equal(db, want[2]), case
     if init:
         assert torch.equal(dinit, want[3])
     outside = torch.ones(wide, dtype=torch.bool)
