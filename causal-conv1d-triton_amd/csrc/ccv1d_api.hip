@@ -801,7 +801,9 @@ struct BwdPlan {
 
 // Kernels, tiling and workspace of a backward with these rows (B, T, D > 0): the matrix-core or the
 // vectorised kernels when the x dtype, the width, the channels and the extent of x, dout and dx allow
-// them (rows_ok; any row alignment does), else the generic ones.
+// them (rows_ok; any row alignment does), else the generic ones. `most`: bytes that the partial rows of a
+// fixed workspace may take (0: any). Where 4 channels do not divide the rows and need more, 2 channels
+// per lane are taken, whose longer tiles leave fewer partial rows.
 struct BwdPath {
   bool mfma = false;
   bool fast = false;
@@ -816,7 +818,7 @@ BwdPath bwd_path(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dt
                  const void* dout, int64_t dout_stride_b, int64_t dout_stride_t,
                  const void* dfinal_states, const void* dx, int64_t dx_stride_b,
                  int64_t dx_stride_t, bool ws_aligned, bool mfma, int64_t B, int64_t T, int64_t D,
-                 int64_t W) {
+                 int64_t W, size_t most = 0) {
   BwdPath r;
   r.mfma = mfma && mfma_pays(B, T, D, W, true) && rows_ok(x_dtype, 2, T, D, x, x_stride_t) &&
            rows_ok(x_dtype, 2, T, D, dout, dout_stride_t) &&
@@ -828,13 +830,16 @@ BwdPath bwd_path(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dt
     r.need = partial_bytes(r.rows, W, D);
     return r;
   }
-  const int bcpl = bwd_shape(x_dtype, B, T, D, W).cpl;
+  const FastShape sh = bwd_shape(x_dtype, B, T, D, W);
+  const int bcpl = sh.cpl;
   r.fast = fast_dtype(x_dtype, W) && rows_ok(x_dtype, bcpl, T, D, x, x_stride_t) &&
            rows_ok(x_dtype, bcpl, T, D, dout, dout_stride_t) &&
            rows_ok(x_dtype, bcpl, T, D, dx, dx_stride_t) &&
            (!dfinal_states || aligned_to(dfinal_states, esize(x_dtype))) && ws_aligned;
   if (r.fast) {
     r.tl = bwd_fast_tiling(B, T, D, W, x_dtype, seq);
+    if (most && D % bcpl && partial_bytes(B * r.tl.nTB, W, D) > most)
+      r.tl = bwd_tiling_for(B, T, D, W, x_dtype, cpl_wide(x_dtype), sh.nw, seq);
     r.rows = B * r.tl.nTB;
   } else {
     r.tl = generic_tiling(B, T, D, W, x_dtype, true);
@@ -858,7 +863,7 @@ int plan_bwd(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype,
              const void* dout, int64_t dout_stride_b, int64_t dout_stride_t,
              const void* dfinal_states, void* dx, int64_t dx_stride_b, int64_t dx_stride_t,
              void* dinitial_states, void* dweight, void* dbias, bool ws_aligned, int64_t batch,
-             int64_t seqlen, int64_t dim, int64_t width, int silu, BwdPlan& pl) {
+             int64_t seqlen, int64_t dim, int64_t width, int silu, BwdPlan& pl, size_t most = 0) {
   const int64_t B = batch, T = seqlen, D = dim, W = width;
   int rc = check_common(x, x_stride_b, x_stride_t, x_dtype, weight, weight_dtype, bias, bias_dtype,
                         initial_states, init_dtype, B, T, D, W);
@@ -939,7 +944,7 @@ int plan_bwd(const void* x, int64_t x_stride_b, int64_t x_stride_t, int x_dtype,
                                 dx_stride_t, ws_aligned,
                                 mfma_takes(x_dtype, D, W, silu != 0, seq_idx != nullptr,
                                            initial_states != nullptr, init_dtype),
-                                B, T, D, W);
+                                B, T, D, W, most);
   pl.mfma = path.mfma;
   pl.fast = path.fast;
   pl.wide = path.wide;
@@ -1109,7 +1114,7 @@ int ccv1d_bwd_noalloc(const void* x, int64_t x_stride_b, int64_t x_stride_t, int
   int rc = plan_bwd(x, x_stride_b, x_stride_t, x_dtype, weight, weight_dtype, bias, bias_dtype,
                     seq_idx, initial_states, init_dtype, dout, dout_stride_b, dout_stride_t,
                     dfinal_states, dx, seqlen * dim, dim, dinitial_states, dweight, dbias, true,
-                    batch, seqlen, dim, width, silu, pl);
+                    batch, seqlen, dim, width, silu, pl, CCV1D_NOALLOC_SCRATCH_BYTES);
   if (rc) return rc;
   if (pl.need > (size_t)CCV1D_NOALLOC_SCRATCH_BYTES)
     return fail(CCV1D_ERR_WORKSPACE,

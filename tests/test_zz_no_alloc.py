@@ -122,3 +122,20 @@ def test_no_alloc_against_oracle():
         floor = 1e-5 * ref.pow(2).mean().sqrt().item() + 1e-7
         torch.testing.assert_close(got[key][cols.to(DEV)].double().cpu(), ref, rtol=1e-3,
                                    atol=floor)
+
+
+def test_no_alloc_where_only_longer_tiles_fit():
+    """Rows that 4 channels per lane do not divide and whose partial rows with 4 would exceed the scratch:
+    2 channels per lane, with longer tiles, fit it. dx is the same bits, the sums the same to rounding."""
+    B, T, D, W = 49, 2178, 3850, 4
+    g = torch.Generator(DEV).manual_seed(9)
+    normal = lambda *s, dt=torch.bfloat16: torch.randn(*s, generator=g, device=DEV, dtype=dt)  # noqa: E731
+    t = {"x": normal(B, T, D), "w": normal(D, W, dt=torch.float32) / 2,
+         "b": normal(D, dt=torch.float32), "init": None, "dy": normal(B, T, D), "seq": None}
+    ref = _with_workspace(t)
+    got = _no_alloc(t)
+    assert torch.equal(got["dx"], ref["dx"])
+    for k in ("dw", "db"):
+        r = ref[k]
+        torch.testing.assert_close(got[k], r, rtol=1e-3,
+                                   atol=1e-5 * r.pow(2).mean().sqrt().item() + 1e-7)
